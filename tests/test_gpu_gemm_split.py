@@ -1,0 +1,71 @@
+"""The projections' bf16-matrix-core GEMMs (csrc/gemm_split.hip, products of at
+least 2^24 multiply-adds) against 64-bit sums: partial tiles, k remainders,
+unaligned rows, split-K weight gradients, infinities and NaN.
+
+Bound per element, with S = sum_k |a_k b_k|: the three dropped partial products
+are below 2^-23 S, and each of the K/16 + 4 additions of a sum no larger than S
+rounds by at most 2^-23 S (twice the fp32 unit roundoff, whichever way the
+matrix core rounds)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_dev():
+    import torch
+    assert torch.cuda.is_available()
+    return torch, torch.device("cuda:0")
+
+
+def _check(name, got, a, b, extra=0.0, adds=0):
+    """got against a @ b (+ extra) within the bound of the module docstring; adds: further fp32 additions."""
+    import torch
+    ref = a.double() @ b.double() + extra
+    s = a.double().abs() @ b.double().abs() + (extra.abs() if torch.is_tensor(extra) else extra)
+    bound = 2.0 ** -23 * (1 + a.shape[1] / 16 + 4 + adds) * s
+    bad = (got.double() - ref).abs() > bound
+    assert not bool(bad.any()), f"{name}: {int(bad.sum())} elements past the bound"
+    print(f"  {name} rel {float((got.double() - ref).norm() / ref.norm()):.2e}", flush=True)
+
+
+# (M, N, K): whole 128-wide tiles, one row / column past them, 64-column and
+# few-column outputs, odd k (unaligned rows), a k remainder of 4, few rows
+SHAPES = [(512, 256, 256), (513, 257, 260), (129, 1025, 132), (4100, 64, 64), (700, 36, 1000), (301, 203, 333),
+          (33, 768, 768), (2048, 130, 70)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("pad", [0, 1])
+def test_linear_pair_within_fp32_bound(pkg, torch_dev, M, N, K, pad):
+    torch, dev = torch_dev
+    print(f"gemm split M{M} N{N} K{K} pad{pad}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    # rows of very different sizes: each output row keeps its own precision
+    x = (rnd(M, K) * 10.0 ** torch.linspace(-8, 8, M, device=dev)[:, None])
+    x = torch.nn.functional.pad(x, (0, pad))[:, :K]   # pad: a row stride that is no multiple of four
+    w, b, dy = rnd(N, K), rnd(N), torch.nn.functional.pad(rnd(M, N), (0, pad))[:, :N]
+    _check("y", pkg.linear_fwd(x, w, b), x, w.t().contiguous(), b.double()[None, :], adds=1)
+    _check("dx", pkg.linear_bwd_dx(dy, w), dy, w)
+    dw, db = pkg.linear_bwd_dw(dy, x)
+    _check("dw", dw, dy.t().contiguous(), x, adds=32)
+    _check("db", db[:, None], dy.t().contiguous(), torch.ones(M, 1, device=dev), adds=M)
+
+
+def test_infinities_and_nan_reach_the_outputs_they_should(pkg, torch_dev):
+    torch, dev = torch_dev
+    M, N, K = 300, 256, 256
+    x, w = torch.randn(M, K, device=dev), torch.randn(N, K, device=dev)
+    w[:, 7] = w[:, 7].abs() + 0.5
+    w[:, 9] = 1.0                       # parts below the first are zero: infinity times them
+    x[3, 7], x[5, 9], x[8, 7], x[10, 1] = float("inf"), float("-inf"), float("nan"), 3.0e38
+    x[10, 2], w[:, 1], w[:, 2] = 3.0e38, 2.0, 2.0   # overflows
+    y = pkg.linear_fwd(x, w)
+    assert bool((y[3] == float("inf")).all()) and bool((y[5] == float("-inf")).all())
+    assert bool(torch.isnan(y[8]).all()) and bool((y[10] == float("inf")).all())
+    keep = torch.ones(M, dtype=torch.bool, device=dev)
+    keep[[3, 5, 8, 10]] = False
+    _check("finite rows", y[keep], x[keep], w.t().contiguous())

@@ -10,8 +10,11 @@
 // with A and B given by strides, so the same kernel serves y = X W^T + b,
 // dX = dY W and dW = dY^T X.
 //
-// Tiling: 128 x 128 (or 64 x 128, 64 x 64) output tile per 256-thread block,
-// 2 x 2 waves; 32-deep k stages fetched straight into LDS by buffer loads
+// Products of at least 2^24 multiply-adds run on the bf16 matrix cores
+// (gemm_split.hip); this file has the small ones and the 64-wide per-head ones.
+//
+// Tiling: 64 x 128 or 64 x 64 output tile per 256-thread block, four waves;
+// 32-deep k stages fetched straight into LDS by buffer loads
 // (gemm_dma_kernel), or, where alignment or size rule those out, 16-deep stages
 // staged through registers with the next stage prefetched (gemm_kernel).
 // MFMA rows are output columns n and MFMA columns are output rows m,
@@ -19,7 +22,7 @@
 // as a float4.  Lane group g covers k = 4g..4g+3 of a stage, so one 128-bit LDS
 // read supplies four MFMA steps.  Split-K writes per-split partial tiles that a
 // second kernel sums in a fixed order (deterministic).
-#include "wha_launch.hpp"
+#include "wha_gemm.hpp"
 
 // k depth of one LDS stage: 16 measured ahead of 32 (layer step 1.498 vs 1.505 ms,
 // wave step 0.879 vs 0.888 ms) and 64 (1.525, 0.900 ms)
@@ -39,41 +42,6 @@
 #endif
 
 namespace wha {
-
-namespace {
-// Output columns per block: 64 per wave along n, WN = 2 waves along n (128
-// columns) or WN = 1 (64 columns, for N <= 64: the per-head value projections).
-constexpr int kGBN = 128;
-}
-
-struct GemmArgs {
-  const float* a;
-  int64_t a_sm, a_sk;  // A(m,k) = a[m*a_sm + k*a_sk]
-  const float* b;
-  int64_t b_sn, b_sk;  // B(k,n) = b[n*b_sn + k*b_sk]
-  float* c;
-  int64_t ldc;         // C(m,n) = c[m*ldc + n]  (or the split-K partial [z][M][N])
-  const float* bias;   // [N] or nullptr
-  int M, N, K;
-  int k_chunk;         // k range per split (multiple of the stage depth)
-  bool c_vec;          // c, ldc and c_sb allow 128-bit stores
-  bool accumulate;     // C += result instead of C = result
-  int batch = 1;       // independent GEMMs, operands offset by the strides below
-  int splits = 1;      // blockIdx.z = batch index * splits + split index
-  int64_t a_sb = 0, b_sb = 0, c_sb = 0, bias_sb = 0;
-  bool a_vec = false;  // A's base, batch stride and row stride along its contiguous
-  bool b_vec = false;  // direction are 16-byte multiples (set by gemm_t); same for B
-  // Row sums of A over the k range (A k-contiguous only, i.e. the weight-gradient
-  // GEMM, where they are the bias gradient): rowsum[bt*rowsum_sb + m] = sum_k A(m,k),
-  // written by the blocks of the first column tile; with split-K each split writes
-  // rowsum_part[(bt*splits + split)*M + m] and the reduce adds the splits in order.
-  float* rowsum = nullptr;
-  int64_t rowsum_sb = 0;
-  float* rowsum_part = nullptr;
-  // gemm_dma_kernel: bytes of one batch's A and B that its loads may touch
-  // (the buffer descriptors' extents; set by gemm_dma_ok)
-  uint32_t a_bytes = 0, b_bytes = 0;
-};
 
 
 // Staging of one ROWS x KT operand tile; element (r, k) of the source is
@@ -693,45 +661,36 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
   }
 }
 
+hipError_t gemm_reduce(const GemmArgs& g, const float* ws, hipStream_t stream) {
+  const int64_t total = (int64_t)g.M * g.N * g.batch;
+  if (g.N % 4 == 0)
+    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0,
+                       stream, ws, g);
+  else
+    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
+                       ws, g);
+  return hipGetLastError();
+}
+
 namespace {
 
-// Output tile: the largest of 128 x 128, 64 x 128 that gives at least eight
-// blocks per CU; 64-column tiles when N <= 64, and for N <= 256 when 64 x 128
-// tiles would leave CUs with fewer (same padding, twice the blocks).  Split-K
-// then picks its factor by rounds of resident blocks (gemm_splits; it once
-// aimed for 1024 blocks in powers of two: weight gradients of the layer step
-// 343 -> 328 us, of the wave step 174 -> 166 us with the rounds model).  Both thresholds were swept on the layer and wave
-// steps (tile 256/512/1024 blocks x split 512/1024/2048: 1024/1024 best, layer
-// 1.465 vs 1.501 ms at 512/512, wave 0.865 vs 0.877 ms); with the buffer-load
-// stages the tile threshold moved to 2048 (the 2304 x 768 c_attn forward in
-// 64 x 128 tiles, three full rounds of three blocks per CU: 126 vs 111 TFLOP/s,
-// layer step 1.369 vs 1.400 ms).
+// Output tile: 64 x 128, or 64 x 64 for few columns (the same padding, twice
+// the blocks).  Split-K then picks its factor by rounds of resident blocks
+// (gemm_splits).  Larger products run in gemm_split.hip.
 constexpr int kCUs = 256;
-#ifndef WHA_GEMM_TILE_BLOCKS
-#define WHA_GEMM_TILE_BLOCKS (8 * kCUs)
-#endif
-struct GemmTile {
-  int bm, bn;
-};
-GemmTile gemm_tile(int M, int N, int batch) {
-  auto blocks = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-  if (N <= 64) return {blocks(128, 64) >= WHA_GEMM_TILE_BLOCKS ? 128 : 64, 64};
-  if (blocks(128, kGBN) >= WHA_GEMM_TILE_BLOCKS) return {128, kGBN};
-  if (blocks(64, kGBN) >= WHA_GEMM_TILE_BLOCKS || N > 256) return {64, kGBN};
-  return {64, 64};
-}
+int gemm_bn(int N) { return N > 256 ? 128 : 64; }
 
 #ifndef WHA_GEMM_FIXK
 #define WHA_GEMM_FIXK 128
 #endif
 // Split-K factor: the split count that minimises rounds x (k per split + a fixed
 // per-block cost), where a round is one block per slot (blocks a CU holds at
-// once: 2 for 128 x 128 tiles, 3 for 64 x 128, 5 for 64 x 64, by their VGPRs
-// and LDS), keeping >= min_k k per split.
+// once: 3 for 64 x 128 tiles, 5 for 64 x 64, by their VGPRs and LDS), keeping
+// >= min_k k per split.
 int gemm_splits(int M, int N, int K, int batch, int min_k = 256) {
-  const GemmTile t = gemm_tile(M, N, batch);
-  const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * batch;
-  const int64_t slots = (int64_t)kCUs * (t.bn == 64 ? 5 : t.bm == 128 ? 2 : 3);
+  const int bn = gemm_bn(N);
+  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + bn - 1) / bn) * batch;
+  const int64_t slots = (int64_t)kCUs * (bn == 64 ? 5 : 3);
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int s = 1; s <= 32; ++s) {
@@ -745,7 +704,6 @@ int gemm_splits(int M, int N, int K, int batch, int min_k = 256) {
   }
   return best;
 }
-
 
 // The direct-to-LDS kernel serves y = x W^T + b, dx = dy W and dW = dy^T x
 // (measured at M = 8192 with per-lane global addresses: layer step 1.477 vs
@@ -798,17 +756,8 @@ hipError_t gemm_launch(GemmArgs g, float* ws, int splits, const char* name, hipS
     hipLaunchKernelGGL((gemm_kernel<BM, KT, WN, A_KC, B_KC, true>), grid, dim3(256), 0, stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int64_t total = (int64_t)g.M * g.N * g.batch;
-  if (g.N % 4 == 0)
-    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0,
-                       stream, (const float*)ws, g);
-  else
-    hipLaunchKernelGGL(gemm_splitk_reduce_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
-                       (const float*)ws, g);
-  return hipGetLastError();
+  return gemm_reduce(g, ws, stream);
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---------------------------------------------------------------- 64 x 64 per-head projections
 // The per-head projections of 64-wide heads (the wave attention's value
@@ -954,20 +903,22 @@ hipError_t gemm_t(GemmArgs g, float* ws, const char* name, hipStream_t stream, i
   // 128-bit loads need every row start along the contiguous direction 16-byte aligned
   g.a_vec = aligned16(g.a) && g.a_sb % 4 == 0 && (A_KC ? g.a_sm % 4 == 0 : g.a_sk % 4 == 0);
   g.b_vec = aligned16(g.b) && g.b_sb % 4 == 0 && (B_KC ? g.b_sn % 4 == 0 : g.b_sk % 4 == 0);
-  const GemmTile t = gemm_tile(g.M, g.N, g.batch);
-  const bool bm128 = t.bm == 128;
-  if (t.bn == 64)
-    return bm128 ? gemm_launch<128, WHA_GEMM_KT, 1, A_KC, B_KC>(g, ws, splits, name, stream)
-                 : gemm_launch<64, WHA_GEMM_KT, 1, A_KC, B_KC>(g, ws, splits, name, stream);
-  return bm128 ? gemm_launch<128, WHA_GEMM_KT, 2, A_KC, B_KC>(g, ws, splits, name, stream)
-               : gemm_launch<64, WHA_GEMM_KT, 2, A_KC, B_KC>(g, ws, splits, name, stream);
+  return gemm_bn(g.N) == 64 ? gemm_launch<64, WHA_GEMM_KT, 1, A_KC, B_KC>(g, ws, splits, name, stream)
+                            : gemm_launch<64, WHA_GEMM_KT, 2, A_KC, B_KC>(g, ws, splits, name, stream);
+}
+
+constexpr int kMaxSplits = 32;
+// Split-K factor of the weight gradient (at least 256 of the position sum per split).
+int dw_splits(int N, int K, int M, int batch) {
+  return gemm_split_ok(M, N, K, batch) ? gemm_pick(N, K, M, batch, true, kMaxSplits, 256).splits
+                                       : gemm_splits(N, K, M, batch);
 }
 
 }  // namespace
 
 size_t linear_dw_workspace_floats(int N, int K, int64_t M, int batch) {
   // split-K partials of the [batch][N][K] weight gradient and of the bias gradient
-  const int splits = gemm_splits(N, K, (int)(M > 0x7fffffff ? 0x7fffffff : M), batch);
+  const int splits = dw_splits(N, K, (int)(M > 0x7fffffff ? 0x7fffffff : M), batch);
   const size_t part = splits > 1 ? (size_t)splits * batch * N * (K + 1) : 0;
   return part + 64;
 }
@@ -976,7 +927,8 @@ size_t linear_dw_workspace_floats(int N, int K, int64_t M, int batch) {
 constexpr int kFwdMinK = 64;
 
 size_t linear_fwd_workspace_floats(int M, int N, int K, int batch) {
-  const int splits = gemm_splits(M, N, K, batch, kFwdMinK);
+  const int splits = gemm_split_ok(M, N, K, batch) ? gemm_pick(M, N, K, batch, false, kMaxSplits, kFwdMinK).splits
+                                                   : gemm_splits(M, N, K, batch, kFwdMinK);
   return splits > 1 ? (size_t)splits * batch * M * N : 0;
 }
 
@@ -994,6 +946,9 @@ hipError_t launch_linear_fwd_batched(const float* x, int64_t ldx, int64_t x_sb, 
   g.b_sb = w_sb;
   g.c_sb = y_sb;
   g.bias_sb = b_sb;
+  if (gemm_split_ok(M, N, K, batch))
+    return gemm_split<true, true>(g, gemm_pick(M, N, K, batch, false, ws != nullptr ? kMaxSplits : 1, kFwdMinK), ws,
+                                  "linear_fwd", stream);
   return gemm_t<true, true>(g, ws, "linear_fwd", stream, kFwdMinK);
 }
 
@@ -1013,6 +968,8 @@ hipError_t launch_linear_bwd_dx_batched(const float* dy, int64_t lddy, int64_t d
   g.a_sb = dy_sb;
   g.b_sb = w_sb;
   g.c_sb = dx_sb;
+  if (gemm_split_ok(M, N, K, batch))
+    return gemm_split<true, false>(g, gemm_pick(M, K, N, batch, true, 1, 1), nullptr, "linear_bwd_dx", stream);
   return gemm_t<true, false>(g, nullptr, "linear_bwd_dx", stream);
 }
 
@@ -1030,13 +987,15 @@ hipError_t launch_linear_bwd_dw_batched(const float* dy, int64_t lddy, int64_t d
   g.a_sb = dy_sb;
   g.b_sb = x_sb;
   g.c_sb = dw_sb;
-  const int splits = gemm_splits(N, K, M, batch);
+  const int splits = dw_splits(N, K, M, batch);
   float* part = splits > 1 ? ws : nullptr;
   if (db != nullptr) {
     g.rowsum = db;
     g.rowsum_sb = N;
     if (splits > 1) g.rowsum_part = ws + (size_t)splits * batch * N * K;
   }
+  if (gemm_split_ok(M, N, K, batch))
+    return gemm_split<false, false>(g, gemm_pick(N, K, M, batch, true, kMaxSplits, 256), part, "linear_bwd_dw", stream);
   return gemm_t<false, false>(g, part, "linear_bwd_dw", stream);
 }
 
