@@ -16,8 +16,9 @@
  *     (NULL = the null stream) and return without synchronising.
  *   - Host entry points take host pointers in the reference's per-sequence
  *     layout and return after the results are in host memory.
- *   - All tensors are fp32.  Arithmetic is fp32 throughout (MFMA
- *     v_mfma_f32_16x16x4_f32 for the contractions).
+ *   - All tensors are fp32, and so is the arithmetic: contractions run on fp32
+ *     MFMAs, or on bf16 MFMAs with each fp32 in three exact bf16 parts and six
+ *     products accumulated in fp32, whose error is no larger.
  *   - Entry points are re-entrant and may be called from several host
  *     threads at once (the reference calls the backend from one thread per
  *     batch element, src/cpu/train_loop.rs:320-365).
@@ -100,7 +101,7 @@ int wha_attn_bwd(const float* q, const float* k, const float* v,
  * reference's forward keeps its attention weights and hands them to
  * attention_backward (src/common/compute.rs:391-399 -> :286-314,
  * src/cpu/backward.rs:330).  wha_attn_fwd_keep is wha_attn_fwd that also
- * writes the raw scores q_t.k_j*scale*log2(e) of the causal half into scores;
+ * writes the raw scores q_t.k_j of the causal half into scores;
  * wha_attn_bwd_kept is wha_attn_bwd that reads them instead of recomputing
  * q k^T (same workspace as wha_attn_bwd).  scores: wha_attn_scores_size bytes
  * of device memory, 16-byte aligned, opaque (its layout is internal), valid

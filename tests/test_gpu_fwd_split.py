@@ -1,0 +1,114 @@
+"""The attention forward on the bf16 matrix cores (attn_fwd_split.hip) against 64-bit
+arithmetic, at the edges of its tiles: 32 keys, 128 queries a block, one kernel per head
+dim class (32, 48, 64, 96, 128).
+
+The bound, with u = 2^-24: a score is a sum of D exact-product terms in three-part form,
+the dropped parts below 4u of |q||k|, summed in fp32 in any order, so its error e is at
+most (D + 8) u |q|.|k| scale; the exponent and exp2 add u (|s| + |m|) + 4u.  A row's
+probabilities then move by P (e + mean e), its output by that times |v|, plus the
+rounding of the sums over at most T keys in tiles of 32: (T / 32 + 40) u sum P |v|.
+"""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def exact(q, k, v, scale, adds=None, drop=None):
+    """O, LSE and their bounds, in 64 bits; without key `drop`."""
+    q, k, v = (x.double() for x in (q, k, v))
+    T, D = q.shape[-2:]
+    adds = T / 32 + 40 if adds is None else adds
+    s = (q @ k.transpose(-1, -2).contiguous()) * scale
+    e = (q.abs() @ k.abs().transpose(-1, -2).contiguous()) * scale * (D + 8) * U
+    mask = torch.ones(T, T, dtype=torch.bool, device=q.device).triu(1)
+    if drop is not None:
+        mask[:, drop] = True
+    s = s.masked_fill(mask, -math.inf)
+    lse = torch.logsumexp(s, -1, keepdim=True)
+    p = torch.exp(s - lse)
+    e = e + U * (s.abs().masked_fill(mask, 0) + s.amax(-1, keepdim=True).abs()) + 4 * U
+    pe = p * e
+    mean = pe.sum(-1, keepdim=True)
+    vmag = v.abs()
+    o_tol = pe @ vmag + (mean + adds * U) * (p @ vmag)
+    return p @ v, lse[..., 0], o_tol, (mean + adds * U)[..., 0] + U * lse[..., 0].abs()
+
+
+def check(o, lse, q, k, v, scale):
+    want_o, want_l, tol_o, tol_l = exact(q, k, v, scale)
+    assert ((o.double() - want_o).abs() <= tol_o).all()
+    assert ((lse.double() - want_l).abs() <= tol_l).all()
+
+
+def draw(B, H, T, D, seed, mixed=False):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    q, k, v = (torch.randn(B, H, T, D, device="cuda", generator=g) for _ in range(3))
+    if mixed:  # rows from 2^-12 to 2^2 beside each other, and a common offset
+        e = torch.randint(-12, 3, (3, B, H, T, 1), device="cuda", generator=g).float().exp2()
+        q, k, v = q * e[0], k * e[1] + 0.5, v * e[2] + 3.0
+    return q, k, v
+
+
+@pytest.mark.parametrize("D", [4, 32, 33, 36, 48, 50, 64, 65, 96, 100, 127, 128])
+@pytest.mark.parametrize("T", [513, 640, 671, 1000])
+def test_tile_edges(pkg, T, D):
+    q, k, v = draw(2, 17, T, D, T * 1000 + D, mixed=True)
+    o, lse = pkg.attn_fwd(q, k, v)
+    check(o, lse, q, k, v, 1 / math.sqrt(D))
+    # the element loads (a base 4 bytes off) stage the same tiles: bit-identical
+    parts = []
+    for x in (q, k, v):
+        buf = torch.empty(x.numel() + 4, device="cuda")
+        parts.append(buf[1:1 + x.numel()].view_as(x).copy_(x))
+    o2, lse2 = pkg.attn_fwd(*parts)
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+@pytest.mark.parametrize("D", [48, 64, 128])
+def test_token_major_rows(pkg, D):
+    """[B,T,H,D] memory (row stride H*D), as the layer holds it."""
+    q, k, v = draw(2, 32, 777, D, D)
+    qt, kt, vt = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v))
+    o, lse = pkg.attn_fwd(q, k, v)
+    ot, lset = pkg.attn_fwd(qt, kt, vt)
+    assert torch.equal(o, ot) and torch.equal(lse, lset)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_rows_that_are_not_finite(pkg, D):
+    """A row sees an infinity or NaN of the keys and values up to its own only.  Rows whose
+    32-key tile holds one are summed again key by key: at most T additions, so the bound
+    has T u where it had (T / 32 + 40) u."""
+    T, at, ch = 700, 333, 1
+    q, k, v = draw(3, 32, T, D, 7)
+    o, lse = pkg.attn_fwd(q, k, v)
+    v2 = v.clone()
+    v2[0, 0, at, ch] = math.inf
+    k2 = k.clone()
+    k2[0, 1, at, 0] = math.nan
+    k2[0, 2, at, 0] = math.inf      # a score of -inf where q is negative there: weight 0
+    o2, lse2 = pkg.attn_fwd(q, k2, v2)
+    same = torch.ones_like(lse, dtype=torch.bool)
+    same[0, :3, at // 32 * 32:] = False
+    assert torch.equal(o[same], o2[same]) and torch.equal(lse[same], lse2[same])
+    scale = 1 / math.sqrt(D)
+    want, want_l, tol, tol_l = exact(q[0, :3], k[0, :3], v[0, :3], scale, adds=T)
+    for h in range(3):  # the rows before it
+        assert ((o2[0, h, :at].double() - want[h, :at]).abs() <= tol[h, :at]).all()
+        assert ((lse2[0, h, :at].double() - want_l[h, :at]).abs() <= tol_l[h, :at]).all()
+    assert (o2[0, 0, at:, ch] == math.inf).all()
+    rest = [d for d in range(D) if d != ch]
+    assert ((o2[0, 0].double() - want[0]).abs() <= tol[0])[:, rest].all()
+    assert o2[0, 1, at:].isnan().all() and lse2[0, 1, at:].isnan().all()
+    pos = torch.nonzero(q[0, 2, at:, 0] > 0)[:, 0] + at
+    neg = torch.nonzero(q[0, 2, at:, 0] < 0)[:, 0] + at
+    assert o2[0, 2, pos].isnan().all()
+    want, want_l, tol, tol_l = exact(q[0, 2], k[0, 2], v[0, 2], scale, adds=T, drop=at)
+    assert ((o2[0, 2].double() - want).abs() <= tol)[neg].all()
+    assert ((lse2[0, 2].double() - want_l).abs() <= tol_l)[neg].all()

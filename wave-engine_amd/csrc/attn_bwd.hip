@@ -91,8 +91,8 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const float* __rest
 // (Tb = T rounded up to 32): block j holds -LSE_t*lse_mult for t = 32j..32j+31,
 // then -Delta_t for the same rows (rows past T hold 0).  The key-stationary
 // kernel fetches a block with one 256-byte load and starts its S and dP
-// accumulators from it.  lse_mult is log2(e) when S comes in log2 units (the
-// kept scores: p = exp2(acc)) and 1/scale when S is recomputed from raw Q and
+// accumulators from it.  lse_mult is log2(e) when S is added in log2 units (the
+// kept scores: p = exp2(score * scale*log2(e) + acc)) and 1/scale when S is recomputed from raw Q and
 // K (acc is then in dot-product units and p = exp2(acc * scale*log2(e))).
 // Same 16-lanes-per-row dot product as attn_bwd_delta_kernel.
 __global__ __launch_bounds__(256) void attn_bwd_stats_kernel(const float* __restrict__ O,
@@ -551,8 +551,8 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkv_kernel(
 // key-tile x query-tile products for every block), so equal blocks fill the
 // CUs to the end instead of leaving a tail of short blocks;
 // grid = B*H*ceil(n_kt/2).
-// SAVED: S comes from the forward's kept scores SC (attn_fwd_dma_kernel with
-// SAVE, same layout as DS) instead of Q K^T: a lane's 8 scores of the next
+// SAVED: S comes from the forward's kept scores SC (raw q.k,
+// attn_fwd_split_kernel with SAVE; the layout of DS) instead of Q K^T: a lane's 8 scores of the next
 // sub-tile are loaded while the current one is consumed (two register sets,
 // alternating with the unrolled loop), and K is not needed at all.
 // PROBS (with SAVED): SC is the caller's att [B][H][T][T] and P is read as
@@ -701,6 +701,8 @@ __global__ __launch_bounds__(256) WHA_DMA_WPE(DP) void attn_bwd_dkv_dma_kernel(
     int vrow[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) vrow[i] = (int)((kcol - ds_head) * 4) + arow(4 * g + i) * 256;
+    // the kept scores' key columns are in order at every head dim
+    const int sc_col = (lq - arow(lq)) * 4;
     // SAVED: a lane's scores of sub-tile st (rows 32st+16mt+arow(4g+i), this lane's key)
     auto load_sc = [&](int st, float (&dst)[8]) {
       if constexpr (PROBS) {
@@ -716,7 +718,7 @@ __global__ __launch_bounds__(256) WHA_DMA_WPE(DP) void attn_bwd_dkv_dma_kernel(
         for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            dst[4 * mt + i] = buffer_load_float(rsc, vrow[i], (st * BSUB + 16 * mt) * 256);
+            dst[4 * mt + i] = buffer_load_float(rsc, vrow[i] + sc_col, (st * BSUB + 16 * mt) * 256);
         }
       }
     };
@@ -756,7 +758,8 @@ __global__ __launch_bounds__(256) WHA_DMA_WPE(DP) void attn_bwd_dkv_dma_kernel(
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) s[mt][i] = PROBS ? sc[4 * mt + i] : s[mt][i] + sc[4 * mt + i];
+          for (int i = 0; i < 4; ++i)
+            s[mt][i] = PROBS ? sc[4 * mt + i] : fmaf(sc[4 * mt + i], scale_log2, s[mt][i]);
         }
       }
       // lane element (mt,i): query qb+16mt+arow(4g+i), key krow

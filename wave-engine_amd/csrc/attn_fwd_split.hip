@@ -1,0 +1,380 @@
+// Causal attention forward on the bf16 matrix cores at fp32 precision
+// (wha_split.hpp): o = softmax(q k^T scale, causal) v and the row log-sum-exp,
+// for every problem but the small ones (small_problem).
+//
+// A block takes NW x 32 consecutive queries of one (b,h), a wave 32 of them: Q
+// in registers (split, unscaled), 32-key tiles of K and V split by the whole
+// block into two LDS buffers, one barrier per tile -- while a tile is consumed
+// the next one is split into the other buffer and the one after it is loaded.
+// A wave forms S^T = K Q^T (keys on MFMA rows, its queries on columns): a lane
+// holds 16 keys of one query, its running maximum needs one cross-lane step, and
+// P^T is the B operand of O^T += V^T P^T as it stands.
+//
+// S sums its five small products first, then the four (NKS) large ones, in one
+// accumulator; scale*log2(e) is applied in the exponent.  Each tile's V^T P^T is
+// likewise one accumulator from zero, added to O with its factor in one fused
+// multiply-add per element (no branch that keeps a second copy of O).
+//
+// The low parts of an infinity are NaN, so a row that meets one comes out NaN
+// here; rows whose result is not finite are formed again in plain fp32 at the
+// end (slow_row), which is where infinities, NaN and overflow get the values
+// that the formula gives them.
+//
+// Bound by the matrix cores and the VALU beside them: per 32 x 32 tile and wave
+// at head dim 64, 48 MFMAs (1536 cycles) and about 300 VALU issue slots (1200);
+// the MFMAs are busy 45% of the time at the 2.0 GHz that the power leaves them.
+// The softmax of a tile is therefore issued between the MFMAs of the next one's
+// scores, the staging between those of O (interleave, wha_split.hpp).
+//
+// Forward alone, fp32 MFMA kernel (16 queries per wave, 64 per block) -> this
+// one, us; and the relative error of O against 64 bits:
+//   8 x 12 heads, 1024 x 64       128 -> 87      3.3e-7 -> 1.5e-7
+//   16 x 8 heads, 512 x 48        38.2 -> 29.2   2.7e-7 -> 1.5e-7
+//   4 x 32 heads, 2048 x 128      1074 -> 800    4.5e-7 -> 1.6e-7
+//   3 x 10 heads, 1531 x 56       111 -> 68      3.7e-7 -> 1.6e-7
+//   the same at head dim 50       134 -> 90      4.1e-7 -> 1.4e-7
+//   4 x 16 heads, 700 x 96        101 -> 56      3.4e-7 -> 1.7e-7
+//   8 x 8 heads, 600 x 32         38.0 -> 23.1   2.9e-7 -> 1.3e-7
+//   2 x 32 heads, 333 x 100       41.6 -> 32.5   (fewer blocks than CUs)
+//   1 x 4 heads, 8192 x 64        428 -> 312
+// It was the faster one at every head dim and length tried down to the small
+// problems' limit, so the other is gone.
+#include <type_traits>
+
+#include "wha_launch.hpp"
+#include "wha_split.hpp"
+
+namespace wha {
+
+// Row t of a head in plain fp32 (one wave; keys, then d, over the lanes).
+template <bool SAVE>
+__device__ __forceinline__ void slow_row(const float* q, const float* Kb, const float* Vb, float* o, float* lse,
+                                         __amdgpu_buffer_rsrc_t rsc, int t, const View& L, float sl2, int lane) {
+  auto score = [&](int j) {  // log2 units; -infinity past the diagonal
+    if (j > t) return -INFINITY;
+    const float* k = Kb + (int64_t)j * L.st;
+    float s = 0.f;
+    for (int d = 0; d < L.D; ++d) s = fmaf(q[d] * sl2, k[d], s);
+    return s;
+  };
+  float m = -INFINITY;
+  for (int j0 = 0; j0 <= t; j0 += 64) {
+    const float s = score(j0 + lane);
+    m = fmaxf(m, s);
+    if (SAVE && j0 + lane <= t) {
+      const int at = (int)(((ds_block_row(j0 >> 6, L.T) - j0 + t) * 64 + lane) * 4);
+      buffer_store_float(rsc, s / sl2, at, 0);
+    }
+  }
+  for (int x = 1; x < 64; x *= 2) m = fmaxf(m, xor_shfl(m, x));
+  float l = 0.f, o0 = 0.f, o1 = 0.f;  // d = lane and lane + 64
+  for (int j0 = 0; j0 <= t; j0 += 64) {
+    const float p = fast_exp2(score(j0 + lane) - m);
+    l += j0 + lane <= t ? p : 0.f;
+    for (int x = 0; x < 64 && j0 + x <= t; ++x) {
+      const float px = __shfl(p, x, 64);
+      const float* v = Vb + (int64_t)(j0 + x) * L.st;
+      if (lane < L.D) o0 = fmaf(px, v[lane], o0);
+      if (lane + 64 < L.D) o1 = fmaf(px, v[lane + 64], o1);
+    }
+  }
+  for (int x = 1; x < 64; x *= 2) l += xor_shfl(l, x);
+  if (lane < L.D) o[lane] = o0 / l;
+  if (lane + 64 < L.D) o[lane + 64] = o1 / l;
+  if (lse != nullptr && lane == 0) *lse = fmaf(m, kLn2, logf(l));
+}
+
+// SAVE: also keeps the raw scores q.k of every tile it computes in SC (the
+// layout of the backward's dS workspace, ds_block_row; entries after the
+// diagonal hold whatever the tile gave, the backward masks them).
+template <int NKS, int NDT, int NW, bool VEC, bool SAVE>
+__global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kernel(
+    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ O,
+    float* __restrict__ LSE, float* __restrict__ SC, View L, float sl2) {
+  using T3 = Tile3<NKS, NDT>;
+  constexpr int NT = NW * 64, BM = NW * 32;
+  __shared__ __align__(16) unsigned K0[T3::RSIZE], K1[T3::RSIZE], V0[T3::CSIZE], V1[T3::CSIZE];
+
+  const int BH = L.B * L.H;
+  const int n_qt = (L.T + BM - 1) / BM;
+  const int bh = blockIdx.x % BH;  // B*H a multiple of 8: a head's blocks share an XCD's L2
+  // The longest rows of tiles first.  Where every block is resident at once, two
+  // to a CU, the later ones from the shortest up: a CU's pair then has about the
+  // same work everywhere (16 x 8 heads of 512 x 48: 30.2 -> 29.2 us, kept
+  // 36.5 -> 35.4).
+  const int j = (int)(blockIdx.x / BH), j0 = (256 + BH - 1) / BH;
+  const int qt = NDT <= 2 && n_qt * BH <= 512 && j >= j0 ? j - j0 : n_qt - 1 - j;
+  const int b = bh / L.H, h = bh % L.H;
+  const int64_t base = (int64_t)b * L.sb + (int64_t)h * L.sh;
+  const float* Kb = K + base;
+  const float* Vb = V + base;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = qt * BM + wave * 32, qrow = q0 + (lane & 31);
+
+  const uint32_t bytes = VEC ? (uint32_t)(((int64_t)(L.T - 1) * L.st + L.D) * 4) : 0u;
+  const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(Kb, bytes), rv = buffer_rsrc(Vb, bytes);
+  const int64_t sc_rows = ds_rows(L.T);
+  const __amdgpu_buffer_rsrc_t rsc = buffer_rsrc(SAVE ? SC + (int64_t)bh * sc_rows * 64 : Q,
+                                                 SAVE ? (uint32_t)(sc_rows * 256) : 0u);
+  const int Tp = (L.T + 63) / 64 * 64;
+
+  const int n_kt = (min(L.T, (qt + 1) * BM) + 31) / 32;  // tiles the block sweeps
+  const int n_w = min(n_kt, q0 / 32 + 1);                // tiles with a key before some query of the wave
+  TileLoad<NKS, NDT, 4 * NKS, NT, VEC> kl;
+  TileLoad<NKS, NDT, 8 * NDT, NT, VEC> vl;
+  if (VEC) {
+    kl.init(L.st, L.D, tid);
+    vl.init(L.st, L.D, tid);
+  }
+  // tile kt of K / V into the registers (past the last one: the last again, never used)
+  auto load_k = [&](int kt) { kl.load(rk, Kb, min(kt, n_kt - 1) * 32, L.T, L.D, L.st, tid); };
+  auto load_v = [&](int kt) { vl.load(rv, Vb, min(kt, n_kt - 1) * 32, L.T, L.D, L.st, tid); };
+  auto store_k = [&](unsigned* Kd) { kl.template store<false>(Kd, tid); };
+  auto store_v = [&](unsigned* Vd) { vl.template store<true>(Vd, tid); };
+  Frag3 qf[NKS];
+  load_k(0);
+  load_v(0);
+  load_frags<NKS, VEC>(Q + base, qrow, L.T, L.D, L.st, lane, qf);
+  store_k(K0);
+  load_k(1);
+  __syncthreads();
+  store_k(K1);
+  load_k(2);
+  store_v(V0);
+  load_v(1);
+
+  // running maximum m (log2 units; finite from the first tile on, whose key 0
+  // comes before every query), this lane's part of the row sum, O
+  float m = -INFINITY, l = 0.f;
+  floatx16 o[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = zero16();
+  floatx16 s;
+
+  // The scores of a tile against the wave's queries: MFMA i of 6 NKS, the small
+  // products of every k-step, then the large ones.
+  constexpr int NMS = 6 * NKS, NMO = 12 * NDT;
+  auto score_step = [&](auto ic, const unsigned* Ks, Frag3 (&kf)[NKS], floatx16& acc) {
+    constexpr int i = decltype(ic)::value;
+    if constexpr (i < 5 * NKS) {
+      constexpr int ks = i / 5, e = i % 5;
+      if constexpr (e == 1 && ks + 1 < NKS) kf[ks + 1] = T3::rows_frag(Ks, ks + 1, lane);
+      acc = mfma_small_step(e, kf[ks], qf[ks], acc);
+    } else {
+      acc = mfma_bf16(kf[i - 5 * NKS].h, qf[i - 5 * NKS].h, acc);
+    }
+  };
+  {
+    Frag3 kf[NKS];
+    kf[0] = T3::rows_frag(K0, 0, lane);
+    s = zero16();
+    run_pieces<0, NMS>([&](auto i) { score_step(i, K0, kf, s); });
+  }
+
+  // Tile kt, whose scores s are there: softmax and O.  NEXT: with the scores of
+  // tile kt + 1, whose MFMAs run beside the softmax of tile kt; the staging of
+  // K tile kt + 2 and V tile kt + 1 runs beside the MFMAs of O.  The last tile
+  // of a wave is the only one with keys past a query or the end.
+  auto tile = [&](auto next, int kt, const unsigned* Kn, const unsigned* Vs, unsigned* Kst, unsigned* Vst) {
+    constexpr bool NEXT = decltype(next)::value;
+    const int k0 = kt * 32;
+    if constexpr (SAVE) {
+      // a lane's four quads of 16 bytes lie 32 bytes apart; swapped with the
+      // lane 16 on, four lanes hold 64 contiguous bytes of one row (kept
+      // forward and backward of 16 x 8 heads of 512 x 48: 128.8 -> 126.0 us)
+      const int c = k0 >> 6, r0 = q0 + (lane & 15);
+      const int at =
+          (int)(((ds_block_row(c, L.T) - (int64_t)64 * c + r0) * 64 + (k0 & 63) + 8 * ((lane >> 4) & 1) + 4 * g) * 4);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        floatx4 lo, hi;  // rows r0 and r0 + 16, keys 16u..16u+15
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[8 * u + e]),
+                                                          __float_as_uint(s[8 * u + 4 + e]), false, false);
+          lo[e] = __uint_as_float(x[0]);
+          hi[e] = __uint_as_float(x[1]);
+        }
+        if (r0 < Tp) buffer_store_quad(rsc, lo, at + 64 * u, 0);
+        if (r0 + 16 < Tp) buffer_store_quad(rsc, hi, at + 64 * u + 16 * 256, 0);
+      }
+    }
+    if constexpr (!NEXT) {
+      const int key_last = min(qrow, L.T - 1);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = k0 + acc_row(i, g) > key_last ? -INFINITY : s[i];
+    }
+    // softmax in pieces: the maximum, then pairs of probabilities and their split
+    float mx = 0.f, alpha = 0.f, sum = 0.f, p[16];
+    uintx4 ph[2], pm[2], pl[2];
+    auto softmax = [&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if constexpr (j == 0) {
+        mx = vmax3(vmax3(vmax3(s[0], s[1], s[2]), s[3], s[4]), vmax3(s[5], s[6], s[7]), s[8]);
+      } else if constexpr (j == 1) {
+        mx = vmax3(vmax3(vmax3(mx, s[9], s[10]), s[11], s[12]), vmax3(s[13], s[14], s[15]), s[15]);
+      } else if constexpr (j == 2) {
+        mx = vmax2(m, pair_max32(mx) * sl2);
+        alpha = fast_exp2(m - mx);
+        m = mx;
+      } else if constexpr (j < 19) {
+        constexpr int k = (j - 3) >> 1;
+        if constexpr (((j - 3) & 1) == 0) {
+          p[2 * k] = fast_exp2(fmaf(s[2 * k], sl2, -m));
+          p[2 * k + 1] = fast_exp2(fmaf(s[2 * k + 1], sl2, -m));
+          pin(p[2 * k]);
+          pin(p[2 * k + 1]);
+        } else {
+          sum += p[2 * k] + p[2 * k + 1];
+          pin(sum);
+          const SplitPair x = split_pair(p[2 * k], p[2 * k + 1]);
+          unsigned xh = x.h, xm = x.m, xl = x.l;
+          pin(xh);
+          pin(xm);
+          pin(xl);
+          ph[k >> 2][k & 3] = xh;
+          pm[k >> 2][k & 3] = xm;
+          pl[k >> 2][k & 3] = xl;
+        }
+      } else {
+        l = fmaf(l, alpha, sum);
+      }
+    };
+    constexpr int NPS = 20;
+    floatx16 sn;
+    if constexpr (NEXT) {
+      Frag3 kf[NKS];
+      kf[0] = T3::rows_frag(Kn, 0, lane);
+      sn = zero16();
+      run_pieces<0, 2>(softmax);
+      WHA_FENCE();
+      interleave<NMS, NPS - 2>(
+          [&](auto i) {
+            score_step(i, Kn, kf, sn);
+            pin(sn);
+          },
+          [&](auto j) { softmax(std::integral_constant<int, decltype(j)::value + 2>{}); });
+    } else {
+      run_pieces<0, NPS>(softmax);
+    }
+    Frag3 pf[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      pf[ks] = Frag3{__builtin_bit_cast(bf16x8, ph[ks]), __builtin_bit_cast(bf16x8, pm[ks]),
+                     __builtin_bit_cast(bf16x8, pl[ks])};
+    // O^T[d][query] = alpha O^T + V^T P^T: per d-tile the small products of both
+    // k-steps, then the large ones
+    Frag3 vf[2 * NDT];
+    vf[0] = T3::cols_frag(Vs, 0, 0, lane);
+    floatx16 t[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) t[dt] = zero16();
+    constexpr int PK = decltype(kl)::template kPieces<false>, PV = decltype(vl)::template kPieces<true>;
+    interleave<NMO, PK + PV + 2>(
+        [&](auto ic) {
+          constexpr int i = decltype(ic)::value, dt = i / 12, e = i % 12;
+          if (e == 1) vf[2 * dt + 1] = T3::cols_frag(Vs, dt, 1, lane);
+          if constexpr (e == 6 && dt + 1 < NDT) vf[2 * dt + 2] = T3::cols_frag(Vs, dt + 1, 0, lane);
+          if constexpr (e < 10)
+            t[dt] = mfma_small_step(e % 5, vf[2 * dt + e / 5], pf[e / 5], t[dt]);
+          else
+            t[dt] = mfma_bf16(vf[2 * dt + e - 10].h, pf[e - 10].h, t[dt]);
+          pin(t[dt]);
+          // the d-tile before, four elements per MFMA
+          if constexpr (dt > 0 && e >= 2 && e < 6) {
+#pragma unroll
+            for (int x = 4 * (e - 2); x < 4 * (e - 1); ++x) o[dt - 1][x] = fmaf(o[dt - 1][x], alpha, t[dt - 1][x]);
+          }
+        },
+        [&](auto jc) {
+          constexpr int j = decltype(jc)::value;
+          if constexpr (j < PK)
+            kl.template store_piece<false>(j, Kst, tid);
+          else if constexpr (j == PK)
+            load_k(kt + 3);
+          else if constexpr (j < PK + 1 + PV)
+            vl.template store_piece<true>(j - PK - 1, Vst, tid);
+          else
+            load_v(kt + 2);
+        });
+#pragma unroll
+    for (int x = 0; x < 16; ++x) o[NDT - 1][x] = fmaf(o[NDT - 1][x], alpha, t[NDT - 1][x]);
+    if constexpr (NEXT) s = sn;
+  };
+  auto step = [&](int kt, const unsigned* Kn, const unsigned* Vs, unsigned* Kst, unsigned* Vst) {
+    __syncthreads();  // K tile kt + 1 and V tile kt are in LDS; every wave is done with the other buffers
+    if (kt + 1 < n_w) {
+      tile(std::true_type{}, kt, Kn, Vs, Kst, Vst);
+    } else if (kt < n_w) {
+      tile(std::false_type{}, kt, Kn, Vs, Kst, Vst);
+    } else {  // every key follows every query of the wave
+      store_k(Kst);
+      load_k(kt + 3);
+      store_v(Vst);
+      load_v(kt + 2);
+    }
+  };
+  for (int kt = 0; kt < n_kt; kt += 2) {
+    step(kt, K1, V0, K0, V1);
+    if (kt + 1 < n_kt) step(kt + 1, K0, V1, K1, V0);
+  }
+
+  const float l_sum = pair_sum32(l);
+  float chk = 0.f * l_sum;  // NaN if the row's sum or any of its O is not finite
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) chk = fmaf(o[dt][x], 0.f, chk);
+  const bool ok = chk == 0.f;
+  if (qrow < L.T && ok) {
+    store_cols<NDT, VEC>(O + base + (int64_t)qrow * L.st, L.D, g, o, 1.f / l_sum);
+    if (LSE != nullptr && g == 0) LSE[(int64_t)bh * L.T + qrow] = fmaf(m, kLn2, logf(l_sum));
+  }
+  const uint64_t bad = __builtin_amdgcn_ballot_w64(qrow < L.T && !ok);
+  for (uint32_t rows = (uint32_t)(bad | (bad >> 32)); rows != 0; rows &= rows - 1) {
+    const int t = q0 + __builtin_ctz(rows);
+    const int64_t at = base + (int64_t)t * L.st;
+    slow_row<SAVE>(Q + at, Kb, Vb, O + at, LSE == nullptr ? nullptr : LSE + (int64_t)bh * L.T + t, rsc, t, L, sl2,
+                   lane);
+  }
+}
+
+namespace {
+template <int NKS, int NDT, int NW>
+void fwd_t(const float* q, const float* k, const float* v, float* o, float* lse, float* sc, const View& L, bool vec,
+           float sl2, hipStream_t stream) {
+  const dim3 grid((unsigned)((int64_t)((L.T + 32 * NW - 1) / (32 * NW)) * L.B * L.H));
+  if (sc != nullptr)
+    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, true>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
+                       lse, sc, L, sl2);
+  else if (vec)
+    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, false>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
+                       lse, sc, L, sl2);
+  else
+    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, false, false>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
+                       lse, sc, L, sl2);
+}
+}  // namespace
+
+hipError_t launch_attn_fwd_split(const float* q, const float* k, const float* v, float* o, float* lse, float* sc,
+                                 const View& L, bool vec, float scale, hipStream_t stream) {
+  // 32-bit byte offsets within a head's rows; otherwise the 64-bit element loads
+  vec = vec && L.D % 4 == 0 && (int64_t)L.T * L.st * 4 < ((int64_t)1 << 31);
+  if (sc != nullptr && !vec) return hipErrorInvalidValue;
+  const float sl2 = (float)((double)scale * 1.4426950408889634);
+  TimingScope ts("attn_fwd", stream);
+  if (L.D <= 32)
+    fwd_t<2, 1, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+  else if (L.D <= 48)
+    fwd_t<3, 2, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+  else if (L.D <= 64)
+    fwd_t<4, 2, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+  else if (L.D <= 96)
+    fwd_t<6, 3, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+  else
+    fwd_t<8, 4, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+  return hipGetLastError();
+}
+
+}  // namespace wha

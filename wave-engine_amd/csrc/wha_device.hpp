@@ -18,11 +18,7 @@
 #ifndef WHA_LDS_PAD
 #define WHA_LDS_PAD 4
 #endif
-// Waves per block of the forward and query-stationary backward kernels
-// (16 queries per wave).
-#ifndef WHA_FWD_NW
-#define WHA_FWD_NW 4
-#endif
+// Waves per block of the query-stationary backward kernel (16 queries per wave).
 #ifndef WHA_DQ_NW
 #define WHA_DQ_NW 4
 #endif
@@ -47,12 +43,10 @@ namespace wha {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
-// The MFMA accumulates a chain of fused multiply-adds, so scores are formed
-// from accumulators started near the row's running maximum (partial sums stay
-// small).  A tile or chunk whose scores pass the maximum it started from by
-// more than this (log2 units) is formed again from the new maximum (the
-// register-staged and small-problem forwards; the direct-to-LDS forward does
-// so in its rescale branch, whose threshold is the same).
+// The fp32 MFMA accumulates a chain of fused multiply-adds, so the small-problem
+// forward forms scores from accumulators started near the row's running maximum
+// (partial sums stay small); a tile whose scores pass the maximum it started
+// from by more than this (log2 units) is formed again from the new maximum.
 constexpr float kRedoMax = 8.f;
 constexpr float kLn2 = 0.69314718055994531f;
 

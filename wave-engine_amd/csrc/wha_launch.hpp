@@ -65,10 +65,14 @@ struct TimingScope {
 };
 
 // Fused forward.  scores != nullptr (only where scores_kept(L, vec)): also
-// writes the raw scores q.k*scale*log2(e) of the causal half into it, in the
-// layout of the dS buffer (bwd_ds_floats(L) floats).
+// writes the raw scores q.k of the causal half into it, in the layout of the dS
+// buffer (bwd_ds_floats(L) floats).
 hipError_t launch_attn_fwd(const float* q, const float* k, const float* v, float* o, float* lse,
                            const View& L, bool vec, float scale, hipStream_t stream, float* scores = nullptr);
+
+// The same on the bf16 matrix cores (attn_fwd_split.hip), any head dim up to 128.
+hipError_t launch_attn_fwd_split(const float* q, const float* k, const float* v, float* o, float* lse, float* scores,
+                                 const View& L, bool vec, float scale, hipStream_t stream);
 
 // The small-problem kernels (attn_small.hip): forward, and the backward in one
 // launch (dK and dV key-stationary, dQ query-stationary with S and dP

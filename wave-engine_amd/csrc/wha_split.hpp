@@ -28,6 +28,8 @@
 // The contraction index k can be mapped to any physical index as long as A and
 // B agree.
 #pragma once
+#include <type_traits>
+
 #include "wha_device.hpp"
 
 namespace wha {
@@ -82,11 +84,234 @@ __device__ __forceinline__ floatx16 mfma_small(const Frag3& a, const Frag3& b, f
   c = mfma_bf16(a.m, b.h, c);
   return mfma_bf16(a.h, b.m, c);
 }
+// Product e (0..4) of mfma_small.
+__device__ __forceinline__ floatx16 mfma_small_step(int e, const Frag3& a, const Frag3& b, floatx16 c) {
+  return e == 0   ? mfma_bf16(a.l, b.h, c)
+         : e == 1 ? mfma_bf16(a.h, b.l, c)
+         : e == 2 ? mfma_bf16(a.m, b.m, c)
+         : e == 3 ? mfma_bf16(a.m, b.h, c)
+                  : mfma_bf16(a.h, b.m, c);
+}
+// Keeps the computation of x where it stands in program order, between the
+// fences around it: an empty statement (no instruction) that x passes through.
+// The optimizer otherwise moves a pure MFMA or VALU chain to its first use.
+template <class T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+// NM MFMAs, mfma(i), with NP pieces of other work, piece(j), spread evenly
+// between them in program order.  A wave issues in order, so only work placed
+// right behind an MFMA runs beside it: up to six VALU operations per MFMA are
+// free there (36 cycles per MFMA against 36 without, measured), in a block after
+// the MFMAs none are -- neither the compiler's order nor a second wave on the
+// SIMD overlapped them.
+template <int J, int END, class P>
+__device__ __forceinline__ void run_pieces(P&& piece) {
+  if constexpr (J < END) {
+    piece(std::integral_constant<int, J>{});
+    run_pieces<J + 1, END>(piece);
+  }
+}
+template <int NM, int NP, int I = 0, class M, class P>
+__device__ __forceinline__ void interleave(M&& mfma, P&& piece) {
+  if constexpr (I < NM) {
+    mfma(std::integral_constant<int, I>{});
+    run_pieces<I * NP / NM, (I + 1) * NP / NM>(piece);
+    WHA_FENCE();
+    interleave<NM, NP, I + 1>(mfma, piece);
+  }
+}
 __device__ __forceinline__ floatx16 zero16() {
   floatx16 z;
 #pragma unroll
   for (int i = 0; i < 16; ++i) z[i] = 0.f;
   return z;
+}
+
+// Row within a 32 x 32 MFMA result of element i of lane group g.
+__device__ __forceinline__ int acc_row(int i, int g) { return 8 * (i >> 2) + 4 * g + (i & 3); }
+
+// A 32-row tile of a [T][D] operand in LDS, as three bf16 planes, in one of two
+// layouts:
+//   rows  [32][16 NKS d]: operand of contractions over the head dimension
+//         (k-slot s of k-step ks is d = 16 ks + s).  Row pitch an odd number of
+//         quads, so any 16 lanes reading the same quad of rows distinct mod 16
+//         (the sets the LDS serves together) meet 16 different quads.
+//   cols  [32 NDT d][32 slots]: operand of contractions over the tile's rows.
+//         Slot 8g + j of k-step ks is row 16 ks + acc_row(j, g), the order in
+//         which a lane holds the elements of a 32 x 32 MFMA result -- which is
+//         so the other operand as it stands, without a shuffle.  d = 4q + u is
+//         stored at row (8 NDT) u + q, quad c at c ^ ((q >> 2) ^ u) & 3: reads
+//         and stores (below) are free of bank conflicts.
+// A staging unit is two adjacent rows x 4 d, two 128-bit loads; unit x is
+// d-group x % G of row pair x / G, pairs ordered so that four consecutive ones
+// fill one quad of cols.
+template <int NKS, int NDT>
+struct Tile3 {
+  static constexpr int RP = 4 * (2 * NKS | 1);  // rows pitch (dwords)
+  static constexpr int RPLANE = 32 * RP, CPLANE = 32 * NDT * 16;
+  static constexpr int RSIZE = 3 * RPLANE, CSIZE = 3 * CPLANE;
+
+  __device__ __forceinline__ static int pair_row(int jj) {
+    return 16 * (jj >> 3) + 8 * ((jj >> 1) & 1) + 4 * ((jj >> 2) & 1) + 2 * (jj & 1);
+  }
+  // dword offset in a rows plane of d = 4q .. 4q + 3 of row r
+  __device__ __forceinline__ static int rows_at(int r, int q) { return r * RP + 2 * q; }
+  // dword offset in a cols plane of row pair jj of d = 4q + u
+  __device__ __forceinline__ static int cols_at(int q, int u, int jj) {
+    const int c = 2 * (jj >> 3) + ((jj >> 2) & 1);
+    return (8 * NDT * u + q) * 16 + 4 * (c ^ (((q >> 2) ^ u) & 3)) + (jj & 3);
+  }
+  __device__ __forceinline__ static Frag3 read(const unsigned* p, int plane) {
+    return Frag3{*reinterpret_cast<const bf16x8*>(p), *reinterpret_cast<const bf16x8*>(p + plane),
+                 *reinterpret_cast<const bf16x8*>(p + 2 * plane)};
+  }
+  __device__ __forceinline__ static const unsigned* rows_ptr(const unsigned* t, int ks, int lane) {
+    return t + (lane & 31) * RP + 4 * (2 * ks + (lane >> 5));
+  }
+  __device__ __forceinline__ static Frag3 rows_frag(const unsigned* t, int ks, int lane) {
+    return read(rows_ptr(t, ks, lane), RPLANE);
+  }
+  // d = 32 dt + lane % 32
+  __device__ __forceinline__ static const unsigned* cols_ptr(const unsigned* t, int dt, int ks, int lane) {
+    const int d = 32 * dt + (lane & 31), q = d >> 2, u = d & 3;
+    return t + (8 * NDT * u + q) * 16 + 4 * ((2 * ks + (lane >> 5)) ^ (((q >> 2) ^ u) & 3));
+  }
+  __device__ __forceinline__ static Frag3 cols_frag(const unsigned* t, int dt, int ks, int lane) {
+    return read(cols_ptr(t, dt, ks, lane), CPLANE);
+  }
+};
+
+// Staging registers of one operand tile for NT threads: G d-groups of 4.
+template <int NKS, int NDT, int G, int NT, bool VEC>
+struct TileLoad {
+  using T3 = Tile3<NKS, NDT>;
+  static constexpr int UNITS = 16 * G, PER = (UNITS + NT - 1) / NT;
+  float v[PER][2][4];
+  uint32_t off[PER];  // VEC: byte offset of the unit's first row at tile row 0
+
+  __device__ __forceinline__ static int unit(int p, int tid) { return (tid + p * NT) % UNITS; }
+  __device__ __forceinline__ void init(int64_t st, int D, int tid) {
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int x = unit(p, tid), c = 4 * (x % G);
+      // past the head dim: an offset past any descriptor's range reads as zero
+      off[p] = c < D ? (uint32_t)(T3::pair_row(x / G) * st + c) * 4u : 0x80000000u;
+    }
+  }
+  // Rows row0 .. row0+31 of the head's rows (zero past T and D).  VEC: through
+  // the head's descriptor ((T-1)*st + D floats, below 2 GiB).
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, const float* base, int row0, int T, int D,
+                                       int64_t st, int tid) {
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      if (VEC) {
+        const uint32_t o = off[p] + (uint32_t)(row0 * st) * 4u;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const float4 x = buffer_load_quad(rsrc, (int)(o + (uint32_t)(r * st) * 4u), 0);
+          v[p][r][0] = x.x, v[p][r][1] = x.y, v[p][r][2] = x.z, v[p][r][3] = x.w;
+        }
+      } else {
+        const int x = unit(p, tid), c = 4 * (x % G), r0 = row0 + T3::pair_row(x / G);
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[p][r][e] = (r0 + r < T && c + e < D) ? base[(int64_t)(r0 + r) * st + c + e] : 0.f;
+      }
+    }
+  }
+  // Splits the units into the planes of one layout (COLS: cols, else rows), in
+  // pieces of three to eight VALU operations.
+  float m[2][4], l[2][4];
+  template <bool COLS>
+  static constexpr int kPieces = PER * (COLS ? 8 : 6);
+  template <bool COLS>
+  __device__ __forceinline__ void store_piece(int j, unsigned* tile, int tid) {
+    constexpr int UP = COLS ? 8 : 6;
+    const int p = j / UP, e = j % UP;
+    const int x = unit(p, tid), q = x % G, jj = x / G, r0 = T3::pair_row(jj);
+    if (e < 4) {
+      const int r = e >> 1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (e & 1) {
+          l[r][i] = m[r][i] - top16(m[r][i]);
+        } else {
+          if constexpr (NDT > 2) pin(v[p][r][i]);  // not before: the load has until here (costs registers)
+          m[r][i] = v[p][r][i] - top16(v[p][r][i]);
+        }
+      }
+    } else if (!COLS) {
+      static_assert(COLS || G == 4 * NKS, "a d-group per quad of a row");
+      const int r = e - 4;
+      unsigned* d = tile + T3::rows_at(r0 + r, q);
+      const float* h = v[p][r];
+      *reinterpret_cast<uintx2*>(d) = uintx2{pack_hi16(h[0], h[1]), pack_hi16(h[2], h[3])};
+      *reinterpret_cast<uintx2*>(d + T3::RPLANE) = uintx2{pack_hi16(m[r][0], m[r][1]), pack_hi16(m[r][2], m[r][3])};
+      *reinterpret_cast<uintx2*>(d + 2 * T3::RPLANE) = uintx2{pack_hi16(l[r][0], l[r][1]), pack_hi16(l[r][2], l[r][3])};
+    } else {
+      const int u = e - 4;
+      unsigned* d = tile + T3::cols_at(q, u, jj);
+      d[0] = pack_hi16(v[p][0][u], v[p][1][u]);
+      d[T3::CPLANE] = pack_hi16(m[0][u], m[1][u]);
+      d[2 * T3::CPLANE] = pack_hi16(l[0][u], l[1][u]);
+    }
+  }
+  template <bool COLS>
+  __device__ __forceinline__ void store(unsigned* tile, int tid) {
+    run_pieces<0, kPieces<COLS>>([&](auto j) { store_piece<COLS>(j, tile, tid); });
+  }
+};
+
+// A wave's 32 rows as the other operand of contractions over the head
+// dimension: lane l holds d = 16 ks + 8 (l/32) + j of row `row`, split (zero
+// past T and D).
+template <int NKS, bool VEC>
+__device__ __forceinline__ void load_frags(const float* __restrict__ base, int row, int T, int D, int64_t st, int lane,
+                                           Frag3 (&f)[NKS]) {
+  const float* src = base + (int64_t)min(row, T - 1) * st;
+  float x[NKS][8];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    const int c = 16 * ks + 8 * (lane >> 5);
+    if (VEC) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < T && c + 4 * h < D) v = *reinterpret_cast<const float4*>(src + c + 4 * h);
+        x[ks][4 * h] = v.x, x[ks][4 * h + 1] = v.y, x[ks][4 * h + 2] = v.z, x[ks][4 * h + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[ks][j] = (row < T && c + j < D) ? src[c + j] : 0.f;
+    }
+  }
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) f[ks] = split_frag(x[ks]);
+}
+
+// Writes a lane's part of a result X^T[d][row] (d = 32 dt + acc_row(i, g)) to
+// its row of a [T][D] tensor.
+template <int NDT, bool VEC>
+__device__ __forceinline__ void store_cols(float* __restrict__ dst, int D, int g, const floatx16 (&x)[NDT], float mul) {
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = 32 * dt + 8 * u + 4 * g;
+      if (VEC) {
+        if (c < D)
+          *reinterpret_cast<float4*>(dst + c) = make_float4(x[dt][4 * u] * mul, x[dt][4 * u + 1] * mul,
+                                                            x[dt][4 * u + 2] * mul, x[dt][4 * u + 3] * mul);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < D) dst[c + e] = x[dt][4 * u + e] * mul;
+      }
+    }
 }
 
 }  // namespace wha
