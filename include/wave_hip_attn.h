@@ -345,13 +345,14 @@ int wha_wave_bwd(const float* x, const float* d_out, const wha_wave_weights* w, 
 int wha_wave_probs_rows(const wha_wave_cache* cache, const wha_wave_shape* shape, const int32_t* rows,
                         int32_t n_rows, float* out, void* stream);
 
-/* Kernel family of wha_wave_fwd / wha_wave_bwd, process-wide (no counterpart
+/* Kernel family of wha_wave_fwd / wha_wave_bwd / wha_wave_kv_prefill,
+ * process-wide (no counterpart
  * in the reference; for tests and benchmarks).  mode 1 = bucket-sparse: every
  * (b,h)'s positions sorted by bucket, scores computed only in the 16 x 16
  * blocks the bucket mask can admit, the previous-position term added per
  * query; 0 = every causal pair scored and the mask applied per score;
- * 2 (the default) = bucket-sparse for T >= 1024, where it is measured no
- * slower, all pairs below.  Both give the reference's results within fp32
+ * 2 (the default) = bucket-sparse for T >= 1024 (prefill at head dims outside
+ * 49..64: T >= 2048), where it is measured no slower, all pairs below.  Both give the reference's results within fp32
  * rounding; the sparse family needs up to twice the score-gradient workspace,
  * which wha_wave_bwd_workspace_size always includes.  Returns the previous
  * mode, or -1 (mode unchanged) for a mode outside 0..2. */
@@ -395,7 +396,10 @@ typedef struct wha_wave_kv_cache {
   int32_t capacity;
 } wha_wave_kv_cache;
 
-/* Workspace bytes of wha_wave_kv_prefill for prompts of shape->T positions. */
+/* Workspace bytes of wha_wave_kv_prefill for prompts of shape->T positions,
+ * with the bucket-sparse family's sorted copies (4 bytes x (34 + a few) per
+ * position and head) where the shape can take that family; a workspace without
+ * room for those is accepted and scores every causal pair. */
 size_t wha_wave_kv_prefill_workspace_size(const wha_wave_shape* shape);
 
 /* prefill's attention (kv_cache.rs:121-193) over prompts x [B][T][n_embd]

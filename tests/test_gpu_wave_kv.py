@@ -114,3 +114,38 @@ def test_decode_rejects_a_full_cache(pkg, torch_dev):
     cache.lengths = [4]
     with pytest.raises(pkg.WaveHipError):
         pkg.forward_one_attention(W, torch.zeros(1, E, device=dev), cache)
+
+
+@pytest.mark.parametrize("E,H,T", [(128, 2, 1024), (120, 2, 1531), (64, 2, 2047), (96, 2, 2048), (256, 2, 2049),
+                                   (84, 2, 17)])
+def test_prefill_families_agree(pkg, torch_dev, E, H, T):
+    """Bucket-sparse and all-pairs prefill: the same cache bits, and outputs within fp32
+    rounding.  A row's output is a sum of at most T + 1 weighted values, so two orders of
+    summation differ by at most 2 (T + E) u times the largest value (through out_proj: times
+    its row sums), scores included (|score| <= 1: one feature pair); a workspace without the
+    sorted copies takes all pairs."""
+    import ctypes
+    torch, dev = torch_dev
+    w, W = _weights(pkg, torch, dev, H, 16, E, seed=T)
+    x = torch.from_numpy(np.random.default_rng(T).normal(size=(2, T, E)).astype(np.float32)).to(dev)
+    L = pkg.lib()
+    size = L.wha_wave_kv_prefill_workspace_size(ctypes.byref(pkg.WaveShape(2, T, E, H, 16)))
+    sorted_copies = L.wha_wave_fwd_workspace_size(ctypes.byref(pkg.WaveShape(2, T, E, H, 16)))
+    res = {}
+    for name, mode, n in (("pairs", 0, size), ("sparse", 1, size), ("short", 1, size - sorted_copies), ("own", 2, size)):
+        cache = pkg.WaveKvCache(2, H, E // H, T, dev)
+        ws = torch.full((n // 4,), float("nan"), device=dev)
+        old = L.wha_wave_set_bucket_sparse(mode)
+        try:
+            out = pkg.prefill_attention(W, x, cache, workspace=ws)
+        finally:
+            L.wha_wave_set_bucket_sparse(old)
+        torch.cuda.synchronize()
+        res[name] = (out, cache.values, cache.phase, cache.cs, cache.bucket)
+    assert torch.equal(res["short"][0], res["pairs"][0])
+    assert torch.equal(res["own"][0], res["sparse" if T >= (1024 if 48 < E // H <= 64 else 2048) else "pairs"][0])
+    for a, b in zip(res["pairs"][1:], res["sparse"][1:]):
+        assert torch.equal(a, b)
+    vmax = float(res["pairs"][1].abs().max())
+    bound = 2 * (T + E) * 2.0 ** -24 * vmax * float(np.abs(w["out_w"]).sum(1).max())
+    assert float((res["pairs"][0] - res["sparse"][0]).abs().max()) <= bound

@@ -693,9 +693,9 @@ int wha_wave_set_bucket_sparse(int mode) {
 static bool wave_sparse_fits(const wha_wave_shape* sh) {
   return wha::wave_sparse_ds_floats(sh->B, sh->n_head, sh->T) * sizeof(float) <= kMaxDsBytes;
 }
-static bool wave_sparse_on(const wha_wave_shape* sh) {
+static bool wave_sparse_on(const wha_wave_shape* sh, int min_t = kWaveSparseMinT) {
   const int mode = g_wave_sparse.load(std::memory_order_relaxed);
-  return (mode == 1 || (mode == 2 && sh->T >= kWaveSparseMinT)) && wave_sparse_fits(sh);
+  return (mode == 1 || (mode == 2 && sh->T >= min_t)) && wave_sparse_fits(sh);
 }
 
 // Scratch of the bucket-sparse forward (sorted operand copies), in bytes; 0
@@ -1048,7 +1048,7 @@ static int check_kv(const wha_wave_kv_cache* kv, const char* fn) {
 }
 
 struct KvPrefillParts {
-  size_t proj, values, feat, phase, bucket, merged, lse, total;
+  size_t proj, values, feat, phase, bucket, merged, lse, dense, total;
 };
 
 static KvPrefillParts kv_prefill_parts(const wha_wave_shape* sh) {
@@ -1062,7 +1062,8 @@ static KvPrefillParts kv_prefill_parts(const wha_wave_shape* sh) {
   p.bucket = r64(B * H * T);
   p.merged = r64(B * T * E);
   p.lse = r64(B * H * T);
-  p.total = p.proj + p.values + p.feat + p.phase + p.bucket + p.merged + p.lse;
+  p.dense = p.proj + p.values + p.feat + p.phase + p.bucket + p.merged + p.lse;
+  p.total = p.dense + wave_fwd_sparse_bytes(sh) / sizeof(float);
   return p;
 }
 
@@ -1083,7 +1084,19 @@ int wha_wave_kv_prefill(const float* x, const wha_wave_weights* w, const wha_wav
   hipStream_t s = static_cast<hipStream_t>(stream);
   const KvPrefillParts parts = kv_prefill_parts(shape);
   void* wsv = nullptr;
-  if ((rc = resolve_workspace(workspace, workspace_bytes, parts.total * sizeof(float), s, fn, &wsv))) return rc;
+  // The bucket-sparse forward, which sorts first, from the length at which it is
+  // the faster (whole call, all pairs -> sparse, us): head dim 64, where the
+  // one-wave kernel serves it, 4 x 12 heads of 768 positions 127 -> 128, 1024:
+  // 153 -> 150, 2048: 330 -> 280, 1 x 12 of 4096: 320 -> 257; other head dims
+  // 1 x 8 x 1024 x 48: 79 -> 82, 2 x 32 x 1024 x 128: 665 -> 671, 1 x 4 x 2048 x
+  // 42: 123 -> 116, 2 x 32 x 2048 x 128: 1418 -> 1348.  A workspace without
+  // room for the sorted copies takes all pairs.
+  const int min_t = wha::padded_dim(shape->n_embd / shape->n_head) == 64 ? kWaveSparseMinT : 2 * kWaveSparseMinT;
+  const bool sparse =
+      wave_sparse_on(shape, min_t) && (workspace == nullptr || workspace_bytes >= parts.total * sizeof(float));
+  if ((rc = resolve_workspace(workspace, workspace_bytes, (sparse ? parts.total : parts.dense) * sizeof(float), s, fn,
+                              &wsv)))
+    return rc;
   float* p = static_cast<float*>(wsv);
   float* proj = p;
   p += parts.proj;
@@ -1098,6 +1111,7 @@ int wha_wave_kv_prefill(const float* x, const wha_wave_weights* w, const wha_wav
   float* merged = p;
   p += parts.merged;
   float* lse = p;
+  p += parts.lse;  // the sorted copies
 
   const int B = shape->B, T = shape->T, E = shape->n_embd, H = shape->n_head, C = shape->content_dim;
   const int hd = E / H, HP = H * (2 + C), M = B * T;
@@ -1107,8 +1121,10 @@ int wha_wave_kv_prefill(const float* x, const wha_wave_weights* w, const wha_wav
     e = wha::launch_linear_fwd_batched(x, E, hd, w->v_w, (int64_t)hd * hd, w->v_b, hd, values, E, hd, M, hd, hd, H,
                                        s);
   if (e == hipSuccess) e = wha::launch_wave_features(proj, w->harmonic_raw, feat, phase, bucket, B, H, T, C, 0, s);
+  const bool vec = vec_ok(Lv, {values, merged});
   if (e == hipSuccess)
-    e = wha::launch_wave_fwd(feat, bucket, values, merged, lse, Lv, vec_ok(Lv, {values, merged}), 0.f, s);
+    e = sparse ? wha::launch_wave_fwd_sparse(feat, bucket, values, merged, lse, p, Lv, vec, 0.f, s)
+               : wha::launch_wave_fwd(feat, bucket, values, merged, lse, Lv, vec, 0.f, s);
   if (e == hipSuccess) e = wha::launch_linear_fwd(merged, E, w->out_w, w->out_b, out, E, M, E, E, s);
   if (e == hipSuccess)
     e = wha::launch_wave_kv_write(feat, bucket, phase, values, kv->cs, kv->bucket, kv->phase, kv->values, B, H, T,
