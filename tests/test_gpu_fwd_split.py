@@ -80,6 +80,34 @@ def test_token_major_rows(pkg, D):
     assert torch.equal(o, ot) and torch.equal(lse, lset)
 
 
+@pytest.mark.parametrize("D", [48, 128])
+@pytest.mark.parametrize("over", [False, True])
+def test_rows_two_gib_apart(pkg, D, over):
+    """A head's rows up to and past 2 GiB: 32-bit or 64-bit offsets, the same results, kept
+    scores and their backward included."""
+    T = 1061
+    st = ((2 ** 31 // 4) // (T + 32) & ~3) + (4 if over else -4)
+    q, k, v = draw(1, 2, T, D, D)
+    do = draw(1, 2, T, D, D + 1)[0]
+    far = []
+    for x in (q, k, v, do):
+        f = torch.empty(T * st, device="cuda").as_strided((1, 2, T, D), (T * st, D, st, 1))
+        far.append(f.copy_(x))
+    out = []
+    for a in ((q, k, v, do), far):
+        L = pkg.layout_of(a[0])
+        sc = pkg.attn_scores_buffer(L, torch.device("cuda:0"))
+        assert sc is not None
+        o = torch.empty_strided(a[0].shape, a[0].stride(), device="cuda")
+        o, lse = pkg.attn_fwd(a[0], a[1], a[2], out=o, scores=sc)
+        g = [torch.empty_strided(a[0].shape, a[0].stride(), device="cuda") for _ in range(3)]
+        g = pkg.attn_bwd(a[0], a[1], a[2], o, a[3], lse, dq=g[0], dk=g[1], dv=g[2], scores=sc)
+        out.append([x.contiguous() for x in (o, lse, *g)])
+        del o, g, sc
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_rows_that_are_not_finite(pkg, D):
     """A row sees an infinity or NaN of the keys and values up to its own only.  Rows whose

@@ -345,8 +345,11 @@ template <int NKS, int NDT, int NW>
 void fwd_t(const float* q, const float* k, const float* v, float* o, float* lse, float* sc, const View& L, bool vec,
            float sl2, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)((L.T + 32 * NW - 1) / (32 * NW)) * L.B * L.H));
-  if (sc != nullptr)
+  if (sc != nullptr && vec)
     hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, true>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
+                       lse, sc, L, sl2);
+  else if (sc != nullptr)
+    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, false, true>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
                        lse, sc, L, sl2);
   else if (vec)
     hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, false>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
@@ -359,9 +362,9 @@ void fwd_t(const float* q, const float* k, const float* v, float* o, float* lse,
 
 hipError_t launch_attn_fwd_split(const float* q, const float* k, const float* v, float* o, float* lse, float* sc,
                                  const View& L, bool vec, float scale, hipStream_t stream) {
-  // 32-bit byte offsets within a head's rows; otherwise the 64-bit element loads
-  vec = vec && L.D % 4 == 0 && (int64_t)L.T * L.st * 4 < ((int64_t)1 << 31);
-  if (sc != nullptr && !vec) return hipErrorInvalidValue;
+  // 32-bit byte offsets within a head's rows, the last tile's rows past T
+  // included; otherwise the 64-bit element loads
+  vec = vec && L.D % 4 == 0 && ((int64_t)L.T + 32) * L.st * 4 < ((int64_t)1 << 31);
   const float sl2 = (float)((double)scale * 1.4426950408889634);
   TimingScope ts("attn_fwd", stream);
   if (L.D <= 32)
