@@ -1,5 +1,5 @@
 """The projections' bf16-matrix-core GEMMs (csrc/gemm_split.hip, products of at
-least 2^24 multiply-adds) against 64-bit sums: partial tiles, k remainders,
+least 2^24 multiply-adds, weight gradients 2^29) against 64-bit sums: partial tiles, k remainders,
 unaligned rows, split-K weight gradients, infinities and NaN.
 
 Bound per element, with S = sum_k |a_k b_k|: the three dropped partial products
@@ -33,7 +33,7 @@ def _check(name, got, a, b, extra=0.0, adds=0):
 # (M, N, K): whole 128-wide tiles, one row / column past them, 64-column and
 # few-column outputs, odd k (unaligned rows), a k remainder of 4, few rows
 SHAPES = [(512, 256, 256), (513, 257, 260), (129, 1025, 132), (4100, 64, 64), (700, 36, 1000), (301, 203, 333),
-          (33, 768, 768), (2048, 130, 70)]
+          (33, 768, 768), (2048, 130, 70), (4100, 513, 260), (8200, 64, 1028)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

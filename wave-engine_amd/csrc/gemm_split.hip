@@ -432,6 +432,14 @@ GemmPick gemm_pick(int M, int N, int K, int batch, bool rows_contiguous, int max
 bool gemm_split_ok(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return (double)M * (double)N * (double)K * (double)batch >= (double)(1 << 24);
 }
+// Weight gradients from 2^29 on: below, their few output tiles and the split-K
+// sum set the time (us, fp32 MFMA against split, M x N x K: 1024 x 504 x 168
+// 13.7 / 16.5, 4096 x 504 x 168 19.9 / 20.9, 2048 x 384 x 384 21.2 / 21.1, 12
+// heads of 8192 x 64 x 64 16.1 / 22.7; above, 4096 x 768 x 256 26.5 / 27.7, 1024 x
+// 768 x 768 31.9 / 24.4, 8192 x 216 x 768 47.3 / 39.3).
+bool gemm_split_dw_ok(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  return (double)M * (double)N * (double)K * (double)batch >= (double)(1 << 29);
+}
 
 template <bool A_KC, bool B_KC>
 hipError_t gemm_split(const GemmArgs& args, const GemmPick& t, float* ws, const char* name, hipStream_t stream) {

@@ -10,7 +10,7 @@
 // with A and B given by strides, so the same kernel serves y = X W^T + b,
 // dX = dY W and dW = dY^T X.
 //
-// Products of at least 2^24 multiply-adds run on the bf16 matrix cores
+// Products of at least 2^24 multiply-adds (weight gradients 2^29) run on the bf16 matrix cores
 // (gemm_split.hip); this file has the small ones and the 64-wide per-head ones.
 //
 // Tiling: 64 x 128 or 64 x 64 output tile per 256-thread block, four waves;
@@ -910,8 +910,8 @@ hipError_t gemm_t(GemmArgs g, float* ws, const char* name, hipStream_t stream, i
 constexpr int kMaxSplits = 32;
 // Split-K factor of the weight gradient (at least 256 of the position sum per split).
 int dw_splits(int N, int K, int M, int batch) {
-  return gemm_split_ok(M, N, K, batch) ? gemm_pick(N, K, M, batch, true, kMaxSplits, 256).splits
-                                       : gemm_splits(N, K, M, batch);
+  return gemm_split_dw_ok(M, N, K, batch) ? gemm_pick(N, K, M, batch, true, kMaxSplits, 256).splits
+                                          : gemm_splits(N, K, M, batch);
 }
 
 }  // namespace
@@ -994,7 +994,7 @@ hipError_t launch_linear_bwd_dw_batched(const float* dy, int64_t lddy, int64_t d
     g.rowsum_sb = N;
     if (splits > 1) g.rowsum_part = ws + (size_t)splits * batch * N * K;
   }
-  if (gemm_split_ok(M, N, K, batch))
+  if (gemm_split_dw_ok(M, N, K, batch))
     return gemm_split<false, false>(g, gemm_pick(N, K, M, batch, true, kMaxSplits, 256), part, "linear_bwd_dw", stream);
   return gemm_t<false, false>(g, part, "linear_bwd_dw", stream);
 }

@@ -40,11 +40,12 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // Sums the split-K partial tiles ws [batch * splits][M][N] into C (bias, accumulate).
 hipError_t gemm_reduce(const GemmArgs& g, const float* ws, hipStream_t stream);
 
-// gemm_split.hip.  gemm_split_ok: the size rule under which these kernels run.
+// gemm_split.hip.  gemm_split_ok / _dw_ok: the size rules under which these kernels run.
 struct GemmPick {
   int bm, bn, splits;
 };
 bool gemm_split_ok(int64_t M, int64_t N, int64_t K, int64_t batch);
+bool gemm_split_dw_ok(int64_t M, int64_t N, int64_t K, int64_t batch);
 GemmPick gemm_pick(int M, int N, int K, int batch, bool rows_contiguous, int max_splits, int min_k);
 template <bool A_KC, bool B_KC>
 hipError_t gemm_split(const GemmArgs& g, const GemmPick& t, float* ws, const char* name, hipStream_t stream);
