@@ -55,6 +55,19 @@ def test_linear_pair_within_fp32_bound(pkg, torch_dev, M, N, K, pad):
     _check("db", db[:, None], dy.t().contiguous(), torch.ones(M, 1, device=dev), adds=M)
 
 
+@pytest.mark.parametrize("M,N,K", [(700, 36, 1000), (4096, 68, 260)])
+def test_k_remainder_reads_nothing_past_the_operand(pkg, torch_dev, M, N, K):
+    """A last k stage of four rows: the piece past them reads as zero, wherever the memory
+    after the operand lies.  All of it up to 2 GiB on (the lane offset that marks the piece)
+    holds NaN, which a stray read would carry into the sums."""
+    torch, dev = torch_dev
+    buf = torch.full(((1 << 29) + (1 << 20),), float("nan"), device=dev)
+    w = buf[:N * K].view(N, K)             # dx sums over its rows
+    w.copy_(torch.randn(N, K, device=dev))
+    dy = torch.randn(M, N, device=dev)
+    _check("dx", pkg.linear_bwd_dx(dy, w), dy, w.clone())
+
+
 def test_infinities_and_nan_reach_the_outputs_they_should(pkg, torch_dev):
     torch, dev = torch_dev
     M, N, K = 300, 256, 256

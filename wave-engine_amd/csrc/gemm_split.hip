@@ -75,11 +75,12 @@ struct SplitStage {
   }
 
   // Sub-stage s of the stage at k0.  VEC: aligned pieces through the operand's
-  // buffer descriptor (gemm_vec_ok), k past k_end reading as zero (an offset
-  // past the descriptor's range).  Otherwise one predicated load per element.
+  // buffer descriptor (gemm_vec_ok), k past k_end reading as zero (a lane offset
+  // past the descriptor's range; the offset that all lanes share stays on a row
+  // of the operand, K its rows).  Otherwise one predicated load per element.
   template <bool VEC>
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, const float* p, int64_t s_r, int64_t s_k, int r0,
-                                       int R, int k0, int s, int k_end, int tid) {
+                                       int R, int k0, int s, int k_end, int K, int tid) {
     const int k = k0 + 4 * s + kpos(tid);
     if (VEC) {
       const bool past = k >= k_end;  // k_end is a multiple of four, k of KU
@@ -93,7 +94,7 @@ struct SplitStage {
         const int vo = past ? (int)0x80000000 : off[0];
 #pragma unroll
         for (int i = 0; i < KU; ++i) {
-          const int so = (int)((k0 + 4 * s + i) * s_k * 4);
+          const int so = (int)(min(k0 + 4 * s + i, K - 1) * s_k * 4);
           if constexpr (RU == 4) {
             const float4 x = buffer_load_quad(rsrc, vo, so);
             v[s][4 * i + 0] = x.x, v[s][4 * i + 1] = x.y, v[s][4 * i + 2] = x.z, v[s][4 * i + 3] = x.w;
@@ -199,8 +200,8 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
   // (past the last stage the loads start again at stage 0: in bounds, never used)
   auto load = [&](int st, int s) {
     const int k0 = k_begin + (st < nst ? st : 0) * 32;
-    sa.template load<VEC>(ra, A, g.a_sm, g.a_sk, m0, g.M, k0, s, k_end, tid);
-    sb.template load<VEC>(rb, Bm, g.b_sn, g.b_sk, n0, g.N, k0, s, k_end, tid);
+    sa.template load<VEC>(ra, A, g.a_sm, g.a_sk, m0, g.M, k0, s, k_end, g.K, tid);
+    sb.template load<VEC>(rb, Bm, g.b_sn, g.b_sk, n0, g.N, k0, s, k_end, g.K, tid);
   };
   auto store = [&](int s, unsigned* Ad, unsigned* Bd) {
     sa.store(Ad, s, tid);
