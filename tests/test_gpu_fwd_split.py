@@ -3,7 +3,7 @@ arithmetic, at the edges of its tiles: 32 keys, 128 queries a block, one kernel 
 dim class (32, 48, 64, 96, 128).
 
 The bound, with u = 2^-24: a score is a sum of D exact-product terms in three-part form,
-the dropped parts below 4u of |q||k|, summed in fp32 in any order, so its error e is at
+the dropped parts below 1.001 u of |q||k|, summed in fp32 in any order, so its error e is at
 most (D + 8) u |q|.|k| scale; the exponent and exp2 add u (|s| + |m|) + 4u.  A row's
 probabilities then move by P (e + mean e), its output by that times |v|, plus the
 rounding of the sums over at most T keys in tiles of 32: (T / 32 + 40) u sum P |v|.
@@ -68,6 +68,42 @@ def test_tile_edges(pkg, T, D):
         parts.append(buf[1:1 + x.numel()].view_as(x).copy_(x))
     o2, lse2 = pkg.attn_fwd(*parts)
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+def fp32_sums(q, k, v, scale):
+    """O and LSE with every sum a chain of fp32 fused multiply-adds (exact in 64 bits, rounded)."""
+    T, D = q.shape[-2:]
+    s = torch.zeros(*q.shape[:-1], T, device=q.device)
+    for d in range(D):
+        s = (s.double() + q[..., d, None].double() * k[..., None, :, d].double()).float()
+    s = (s * scale).masked_fill(torch.ones(T, T, dtype=torch.bool, device=q.device).triu(1), -math.inf)
+    m = s.amax(-1, keepdim=True)
+    p = torch.exp(s - m)
+    o, l = torch.zeros_like(q), torch.zeros_like(m)
+    for j in range(T):
+        o = (o.double() + p[..., j, None].double() * v[..., j, None, :].double()).float()
+        l = l + p[..., j, None]
+    return o / l, (m + torch.log(l))[..., 0]
+
+
+@pytest.mark.parametrize("kind", ["step", "half"])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_error_no_larger_than_fp32_sums(pkg, D, kind):
+    """Operands where a three-part split does worst (test_gpu_gemm_split.py): the 2-norm error of O
+    and LSE is no larger than that of fp32 sums."""
+    from test_gpu_gemm_split import beside_a_step
+    g = torch.Generator(device="cuda")
+    g.manual_seed(D)
+    q, k, v = (beside_a_step(g, kind, 2, 17, 544, D) for _ in range(3))
+    q = q * (torch.randint(0, 2, q.shape, generator=g, device="cuda").float() * 2 - 1)
+    scale = 1 / math.sqrt(D)
+    o, lse = pkg.attn_fwd(q, k, v)
+    o32, lse32 = fp32_sums(q, k, v, scale)
+    want_o, want_l, _, _ = exact(q, k, v, scale)
+    for name, got, other, want in (("O", o, o32, want_o), ("LSE", lse, lse32, want_l)):
+        e, e32 = ((t.double() - want).norm() / want.norm() for t in (got, other))
+        print(f"  {name} {kind} D {D}: {float(e):.2e}, fp32 sums {float(e32):.2e}", flush=True)
+        assert e <= e32
 
 
 @pytest.mark.parametrize("D", [48, 64, 128])

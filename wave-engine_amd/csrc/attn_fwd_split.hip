@@ -270,7 +270,9 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
     floatx16 t[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) t[dt] = zero16();
-    constexpr int PK = decltype(kl)::template kPieces<false>, PV = decltype(vl)::template kPieces<true>;
+    typename decltype(kl)::Pending kw;
+    typename decltype(vl)::Pending vw;
+    constexpr int PK = decltype(kl)::kPieces, PV = decltype(vl)::kPieces;
     interleave<NMO, PK + PV + 2>(
         [&](auto ic) {
           constexpr int i = decltype(ic)::value, dt = i / 12, e = i % 12;
@@ -290,11 +292,11 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
         [&](auto jc) {
           constexpr int j = decltype(jc)::value;
           if constexpr (j < PK)
-            kl.template store_piece<false>(j, Kst, tid);
+            kl.template store_piece<false>(j, kw, Kst, tid);
           else if constexpr (j == PK)
             load_k(kt + 3);
           else if constexpr (j < PK + 1 + PV)
-            vl.template store_piece<true>(j - PK - 1, Vst, tid);
+            vl.template store_piece<true>(j - PK - 1, vw, Vst, tid);
           else
             load_v(kt + 2);
         });

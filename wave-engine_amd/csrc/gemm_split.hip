@@ -205,6 +205,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
   };
   auto store = [&](int s, unsigned* Ad, unsigned* Bd) {
     sa.store(Ad, s, tid);
+    WHA_FENCE();  // one operand's split at a time: together they spill (128 x 128 weight gradients 137 -> 125 us)
     sb.store(Bd, s, tid);
   };
   auto multiply = [&](const unsigned* Ac, const unsigned* Bc) {
@@ -261,10 +262,11 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
   // C[m][n], m = m0 + 32(MT wm + mt) + lane%32, n = n0 + 32(NT wn + nt) + 8u + 4(lane/32) + e
   const bool vec = PARTIAL ? (g.N % 4 == 0) : g.c_vec;
   const float* bias = (!PARTIAL && g.bias != nullptr) ? g.bias + bt * g.bias_sb : nullptr;
-  // An infinite operand element (its m and l parts are NaN, and infinity times a
-  // zero part is NaN) or a product past the fp32 range makes NaN of sums that
-  // fp32 arithmetic may leave infinite: those elements are summed again in
-  // plain fp32, straight to C, and skipped below.
+  // An infinite operand element, one that rounds to infinity or a product past
+  // the fp32 range leaves infinity or NaN (wha_split.hpp) where fp32 arithmetic
+  // may have another result: those elements are summed again in plain fp32,
+  // straight to C, and skipped below.
+  auto finite = [](float x) { return __builtin_fabsf(x) < INFINITY; };
   bool again = false;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -273,28 +275,28 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         big[nt][mt][i] += small[nt][mt][i];
-        again |= big[nt][mt][i] != big[nt][mt][i];
+        again |= !finite(big[nt][mt][i]);
       }
   auto row_of = [&](int m) {
     return PARTIAL ? g.c + ((int64_t)z * g.M + m) * g.N : g.c + bt * g.c_sb + (int64_t)m * g.ldc;
   };
   if (__builtin_amdgcn_ballot_w64(again) != 0) {
-    uint64_t nan[MT];  // bit 16 nt + i
+    uint64_t redo[MT];  // bit 16 nt + i
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      nan[mt] = 0;
+      redo[mt] = 0;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          nan[mt] |= (uint64_t)(big[nt][mt][i] != big[nt][mt][i]) << (16 * nt + i);
+          redo[mt] |= (uint64_t)!finite(big[nt][mt][i]) << (16 * nt + i);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int m = m0 + 32 * (MT * wm + mt) + (lane & 31);
       for (int x = 0; x < 16 * NT; ++x) {
         const int n = n0 + 32 * (NT * wn + (x >> 4)) + 8 * ((x >> 2) & 3) + 4 * (lane >> 5) + (x & 3);
-        if (!(nan[mt] >> x & 1) || m >= g.M || n >= g.N) continue;
+        if (!(redo[mt] >> x & 1) || m >= g.M || n >= g.N) continue;
         float r = 0.f;
         for (int k = k_begin; k < k_end; ++k)
           r = fmaf(A[(int64_t)m * g.a_sm + (int64_t)k * g.a_sk], Bm[(int64_t)n * g.b_sn + (int64_t)k * g.b_sk], r);
@@ -320,7 +322,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           r[e] = big[nt][mt][4 * u + e];
-          ok[e] = r[e] == r[e] && n + e < g.N;
+          ok[e] = finite(r[e]) && n + e < g.N;
           all &= ok[e];
         }
         float* dst = row + n;

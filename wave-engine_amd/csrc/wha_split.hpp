@@ -1,19 +1,29 @@
 // fp32 contractions on the bf16 matrix cores (gfx950), without giving up fp32
 // precision.
 //
-// An fp32 number is the exact sum of three bf16 numbers: x = h + m + l, where h
-// keeps the sign, the exponent and the top 8 significand bits of x (its upper
-// 16 bits), m the next 8 and l the last 8 (both differences are exact in fp32,
-// and at most 16 and 8 bits wide).  A product x*y is then nine bf16 products,
-// each exact in fp32, of which the MFMA sums the six that reach fp32 precision:
+// An fp32 number is the exact sum of three bf16 numbers (Henry, Tang and
+// Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations", 2019): x = h + m + l, where h is x rounded to
+// bf16, m the difference rounded to bf16 and l what is left (both differences
+// are exact in fp32, |m| <= 2^-8 and |l| <= 2^-17 of x's power of two).  A
+// product x*y is then nine bf16 products, each exact in fp32, of which the MFMA
+// sums the six that reach fp32 precision:
 //   x y = h h' + (h m' + m h') + (h l' + l h' + m m')  + [m l' + l m' + l l']
-// The three left out are below 2^-23 of |x y| together (2^-25 on average); an
-// fp32 sum rounds its result by as much.  The six products go to two
+// The three left out are together below 2^-24 (1 + 2^-10) of |x y|, one fp32
+// rounding, of either sign (2^-28 on average over normal data).  Rounded to
+// nearest, not cut off: the parts of a cut number all have its sign and are up
+// to twice as large, and the three left out reach 2^-21 of every product, all
+// the same way (x = y = 1 + 2^-7 - 2^-23).  The six products go to two
 // accumulators -- h h' to one, the small five to the other -- added once at the
 // end: a small product added to a large accumulator inside the MFMA would lose
 // its low bits at every step (measured over K = 2048 products of one sign: one
 // accumulator 3.5e-6 relative error, two 2.5e-7, the fp32 MFMA 7.0e-7; K = 64
 // of either sign 7.8e-8 against 1.4e-7 of the fp32 MFMA).
+//
+// The upper parts of an infinity leave NaN below them, and so do those of a
+// number from FLT_MAX (1 - 2^-9) on, which rounds to infinity; h h' may also
+// pass the range where the product does not.  A result that is not finite is
+// therefore formed again without the split by each kernel.
 //
 // Why: v_mfma_f32_32x32x16_bf16 does 32768 flops in 32 cycles, v_mfma_f32_16x16x4
 // (fp32) 2048 in 32, so six bf16 products take 0.375 of the fp32 matrix time;
@@ -39,21 +49,29 @@ typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// The three bf16 parts of a pair of floats, each pair packed in one register
-// (first float in the low half).
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// A pair of floats as bf16, to nearest (ties to even), packed in one register
+// (first float in the low half), and what remains of the pair.
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2{a, b}), bf16x2));
+}
+__device__ __forceinline__ unsigned take_pair(float& a, float& b) {
+  const unsigned h = bf16_pair(a, b);
+  a -= __uint_as_float(h << 16);
+  b -= __uint_as_float(h & 0xffff0000u);
+  return h;
+}
+// The three bf16 parts of a pair of floats.
 struct SplitPair {
   unsigned h, m, l;
 };
-__device__ __forceinline__ unsigned pack_hi16(float a, float b) {
-  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
-}
-__device__ __forceinline__ float top16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 __device__ __forceinline__ SplitPair split_pair(float a, float b) {
   SplitPair s;
-  s.h = pack_hi16(a, b);
-  const float am = a - top16(a), bm = b - top16(b);
-  s.m = pack_hi16(am, bm);
-  s.l = pack_hi16(am - top16(am), bm - top16(bm));
+  s.h = take_pair(a, b);
+  s.m = take_pair(a, b);
+  s.l = bf16_pair(a, b);
   return s;
 }
 
@@ -224,45 +242,45 @@ struct TileLoad {
     }
   }
   // Splits the units into the planes of one layout (COLS: cols, else rows), in
-  // pieces of three to eight VALU operations.
-  float m[2][4], l[2][4];
+  // two pieces of five or six VALU operations per pair of elements (a pair is
+  // what a packed register holds: two rows of one d, or two d of one row).
+  struct Pending {  // parts of two pairs, not stored yet
+    uintx2 h, m, l;
+  };
+  static constexpr int kPieces = PER * 8;
   template <bool COLS>
-  static constexpr int kPieces = PER * (COLS ? 8 : 6);
-  template <bool COLS>
-  __device__ __forceinline__ void store_piece(int j, unsigned* tile, int tid) {
-    constexpr int UP = COLS ? 8 : 6;
-    const int p = j / UP, e = j % UP;
-    const int x = unit(p, tid), q = x % G, jj = x / G, r0 = T3::pair_row(jj);
-    if (e < 4) {
-      const int r = e >> 1;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (e & 1) {
-          l[r][i] = m[r][i] - top16(m[r][i]);
-        } else {
-          if constexpr (NDT > 2) pin(v[p][r][i]);  // not before: the load has until here (costs registers)
-          m[r][i] = v[p][r][i] - top16(v[p][r][i]);
-        }
+  __device__ __forceinline__ void store_piece(int j, Pending& w, unsigned* tile, int tid) {
+    const int p = j / 8, k = (j >> 1) & 3;
+    const int x = unit(p, tid), q = x % G, jj = x / G;
+    float& a = COLS ? v[p][0][k] : v[p][k >> 1][2 * (k & 1)];
+    float& b = COLS ? v[p][1][k] : v[p][k >> 1][2 * (k & 1) + 1];
+    if ((j & 1) == 0) {
+      if constexpr (NDT > 2) {  // not before: the load has until here (costs registers)
+        pin(a);
+        pin(b);
       }
-    } else if (!COLS) {
+      w.h[k & 1] = take_pair(a, b);
+      return;
+    }
+    w.m[k & 1] = take_pair(a, b);
+    w.l[k & 1] = bf16_pair(a, b);
+    if (COLS) {
+      unsigned* d = tile + T3::cols_at(q, k, jj);
+      d[0] = w.h[k & 1];
+      d[T3::CPLANE] = w.m[k & 1];
+      d[2 * T3::CPLANE] = w.l[k & 1];
+    } else if (k & 1) {
       static_assert(COLS || G == 4 * NKS, "a d-group per quad of a row");
-      const int r = e - 4;
-      unsigned* d = tile + T3::rows_at(r0 + r, q);
-      const float* h = v[p][r];
-      *reinterpret_cast<uintx2*>(d) = uintx2{pack_hi16(h[0], h[1]), pack_hi16(h[2], h[3])};
-      *reinterpret_cast<uintx2*>(d + T3::RPLANE) = uintx2{pack_hi16(m[r][0], m[r][1]), pack_hi16(m[r][2], m[r][3])};
-      *reinterpret_cast<uintx2*>(d + 2 * T3::RPLANE) = uintx2{pack_hi16(l[r][0], l[r][1]), pack_hi16(l[r][2], l[r][3])};
-    } else {
-      const int u = e - 4;
-      unsigned* d = tile + T3::cols_at(q, u, jj);
-      d[0] = pack_hi16(v[p][0][u], v[p][1][u]);
-      d[T3::CPLANE] = pack_hi16(m[0][u], m[1][u]);
-      d[2 * T3::CPLANE] = pack_hi16(l[0][u], l[1][u]);
+      unsigned* d = tile + T3::rows_at(T3::pair_row(jj) + (k >> 1), q);
+      *reinterpret_cast<uintx2*>(d) = w.h;
+      *reinterpret_cast<uintx2*>(d + T3::RPLANE) = w.m;
+      *reinterpret_cast<uintx2*>(d + 2 * T3::RPLANE) = w.l;
     }
   }
   template <bool COLS>
   __device__ __forceinline__ void store(unsigned* tile, int tid) {
-    run_pieces<0, kPieces<COLS>>([&](auto j) { store_piece<COLS>(j, tile, tid); });
+    Pending w;
+    run_pieces<0, kPieces>([&](auto j) { store_piece<COLS>(j, w, tile, tid); });
   }
 };
 
