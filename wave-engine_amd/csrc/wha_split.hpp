@@ -94,6 +94,11 @@ __device__ __forceinline__ Frag3 split_frag(const float (&x)[8]) {
 __device__ __forceinline__ floatx16 mfma_bf16(bf16x8 a, bf16x8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
+// Two k of fp32 as they stand: lane l supplies A[m = l%32][k = l/32] and
+// B[k = l/32][n = l%32], D as above.
+__device__ __forceinline__ floatx16 mfma_f32(float a, float b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
 // The five small products, smallest first.
 __device__ __forceinline__ floatx16 mfma_small(const Frag3& a, const Frag3& b, floatx16 c) {
   c = mfma_bf16(a.l, b.h, c);
