@@ -179,27 +179,41 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
   auto tile = [&](auto next, int kt, const unsigned* Kn, const unsigned* Vs, unsigned* Kst, unsigned* Vst) {
     constexpr bool NEXT = decltype(next)::value;
     const int k0 = kt * 32;
-    if constexpr (SAVE) {
-      // a lane's four quads of 16 bytes lie 32 bytes apart; swapped with the
-      // lane 16 on, four lanes hold 64 contiguous bytes of one row (kept
-      // forward and backward of 16 x 8 heads of 512 x 48: 128.8 -> 126.0 us)
-      const int c = k0 >> 6, r0 = q0 + (lane & 15);
-      const int at =
-          (int)(((ds_block_row(c, L.T) - (int64_t)64 * c + r0) * 64 + (k0 & 63) + 8 * ((lane >> 4) & 1) + 4 * g) * 4);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        floatx4 lo, hi;  // rows r0 and r0 + 16, keys 16u..16u+15
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[8 * u + e]),
-                                                          __float_as_uint(s[8 * u + 4 + e]), false, false);
-          lo[e] = __uint_as_float(x[0]);
-          hi[e] = __uint_as_float(x[1]);
-        }
-        if (r0 < Tp) buffer_store_quad(rsc, lo, at + 64 * u, 0);
-        if (r0 + 16 < Tp) buffer_store_quad(rsc, hi, at + 64 * u + 16 * 256, 0);
+    // SAVE: quad pair x of the tile's scores (4), among the MFMAs of the next
+    // one's.  A lane's four quads of 16 bytes lie 32 bytes apart; swapped with
+    // the lane 16 on, four lanes hold 64 contiguous bytes of one row (kept
+    // forward and backward of 16 x 8 heads of 512 x 48: 128.8 -> 126.0 us).
+    // Rows past the padded length: an offset past the descriptor, not a branch --
+    // where a store may have been stepped over the compiler waits for all stores
+    // at the next use of a load.  Kept forward, stores under branches before the
+    // MFMAs -> this, us: 4 x 4 heads of 1500 x 48 77.2 -> 65.0, 1 x 2 of 2000 x
+    // 64 103.6 -> 86.4, 1 x 4 of 8192 x 64 433 -> 380, 4 x 32 of 2048 x 128
+    // 943 -> 895, 8 x 12 of 1024 x 64 99.5 -> 100.2 (+-3).
+    int at_lo = 0, at_hi = 0;
+    floatx4 lo, hi;  // rows r0 and r0 + 16, keys 16u .. 16u + 15
+    auto save = [&](auto xc) {
+      constexpr int x = decltype(xc)::value, u = x >> 1;
+      if constexpr (x == 0) {
+        const int c = k0 >> 6, r0 = q0 + (lane & 15);
+        const int at =
+            (int)(((ds_block_row(c, L.T) - (int64_t)64 * c + r0) * 64 + (k0 & 63) + 8 * ((lane >> 4) & 1) + 4 * g) * 4);
+        at_lo = r0 < Tp ? at : (int)0x80000000;
+        at_hi = r0 + 16 < Tp ? at + 16 * 256 : (int)0x80000000;
       }
-    }
+#pragma unroll
+      for (int e = 2 * (x & 1); e < 2 * (x & 1) + 2; ++e) {
+        const auto y = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[8 * u + e]),
+                                                        __float_as_uint(s[8 * u + 4 + e]), false, false);
+        lo[e] = __uint_as_float(y[0]);
+        hi[e] = __uint_as_float(y[1]);
+      }
+      if constexpr (x & 1) {
+        buffer_store_quad(rsc, lo, at_lo + 64 * u, 0);
+        buffer_store_quad(rsc, hi, at_hi + 64 * u, 0);
+      }
+    };
+    constexpr int NPW = SAVE ? 4 : 0;
+    if constexpr (SAVE && !NEXT) run_pieces<0, NPW>(save);
     if constexpr (!NEXT) {
       const int key_last = min(qrow, L.T - 1);
 #pragma unroll
@@ -249,12 +263,18 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
       sn = zero16();
       run_pieces<0, 2>(softmax);
       WHA_FENCE();
-      interleave<NMS, NPS - 2>(
+      interleave<NMS, NPS - 2 + NPW>(
           [&](auto i) {
             score_step(i, Kn, kf, sn);
             pin(sn);
           },
-          [&](auto j) { softmax(std::integral_constant<int, decltype(j)::value + 2>{}); });
+          [&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            if constexpr (j < NPW)
+              save(jc);
+            else
+              softmax(std::integral_constant<int, j - NPW + 2>{});
+          });
     } else {
       run_pieces<0, NPS>(softmax);
     }
