@@ -16,9 +16,9 @@
 // multiply-add per element (no branch that keeps a second copy of O).
 //
 // The low parts of an infinity are NaN, so a row that meets one comes out NaN
-// here; rows whose result is not finite are formed again in plain fp32 at the
-// end (slow_row), which is where infinities, NaN and overflow get the values
-// that the formula gives them.
+// here; rows whose result is not finite are formed again in fp32 at the end
+// (again), which is where infinities, NaN and overflow get the values that the
+// formula gives them.
 //
 // Bound by the matrix cores and the VALU beside them: per 32 x 32 tile and wave
 // at head dim 64, 48 MFMAs (1536 cycles) and about 300 VALU issue slots (1200);
@@ -46,42 +46,120 @@
 
 namespace wha {
 
-// Row t of a head in plain fp32 (one wave; keys, then d, over the lanes).
-template <bool SAVE>
-__device__ __forceinline__ void slow_row(const float* q, const float* Kb, const float* Vb, float* o, float* lse,
-                                         __amdgpu_buffer_rsrc_t rsc, int t, const View& L, float sl2, int lane) {
-  auto score = [&](int j) {  // log2 units; -infinity past the diagonal
-    if (j > t) return -INFINITY;
-    const float* k = Kb + (int64_t)j * L.st;
-    float s = 0.f;
-    for (int d = 0; d < L.D; ++d) s = fmaf(q[d] * sl2, k[d], s);
+// The rows q0 .. q0 + 31 of a head marked in `bad` once more in fp32, straight
+// from memory, by one wave: S^T and O^T on the fp32 MFMA in the layout of the
+// kernel below, the maximum of each row first (an online one would meet
+// -infinity - -infinity), then probabilities and O.  On the last tile some keys
+// follow some queries: there a probability of zero must not meet an infinite
+// value, so its keys are added one at a time to the queries that they precede.
+// All rows NaN or infinite, the whole forward, us: 8 x 12 heads of 1024 x 64 630
+// (one row after another on the VALU 24600; finite 90), 16 x 8 of 512 x 48 231
+// (4870; 35), 4 x 8 of 2048 x 128 2040 (71000; 209).
+template <int NKS, int NDT, bool VEC, bool SAVE>
+__device__ __forceinline__ void again(const float* Qb, const float* Kb, const float* Vb, float* Ob, float* lse,
+                                      __amdgpu_buffer_rsrc_t rsc, int q0, uint32_t bad, const View& L, float sl2,
+                                      int lane) {
+  pin(lane);  // addresses formed from it here, not held in registers since the main loop
+  const int g = lane >> 5, c = lane & 31, qrow = q0 + c, t = min(qrow, L.T - 1), n_w = q0 / 32 + 1;
+  const bool mine = (bad >> c) & 1;
+  // d = 8j + 4g + e of a row (zero past the head dim): k-slot g of MFMA (j, e)
+  auto quad = [&](const float* row, int j, float (&x)[4]) {
+    const int d = 8 * j + 4 * g;
+    if (VEC) {
+      const float4 y = d < L.D ? *reinterpret_cast<const float4*>(row + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+      x[0] = y.x, x[1] = y.y, x[2] = y.z, x[3] = y.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = d + e < L.D ? row[d + e] : 0.f;
+    }
+  };
+  float qf[2 * NKS][4];
+#pragma unroll
+  for (int j = 0; j < 2 * NKS; ++j) {
+    quad(Qb + (int64_t)t * L.st, j, qf[j]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qf[j][e] *= sl2;
+  }
+  // scores of the keys k0 + acc_row(i, g), log2 units
+  auto scores = [&](int k0) {
+    const float* row = Kb + (int64_t)min(k0 + c, L.T - 1) * L.st;
+    floatx16 s = zero16();
+#pragma unroll
+    for (int j = 0; j < 2 * NKS; ++j) {
+      float x[4];
+      quad(row, j, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s = mfma_f32(x[e], qf[j][e], s);
+    }
     return s;
   };
+  auto masked = [&](int k0, int i) { return k0 + acc_row(i, g) > t; };
   float m = -INFINITY;
-  for (int j0 = 0; j0 <= t; j0 += 64) {
-    const float s = score(j0 + lane);
-    m = fmaxf(m, s);
-    if (SAVE && j0 + lane <= t) {
-      const int at = (int)(((ds_block_row(j0 >> 6, L.T) - j0 + t) * 64 + lane) * 4);
-      buffer_store_float(rsc, s / sl2, at, 0);
+  for (int kt = 0; kt < n_w; ++kt) {
+    const int k0 = kt * 32;
+    const floatx16 s = scores(k0);
+    if constexpr (SAVE) {
+      const int at = (int)(((ds_block_row(k0 >> 6, L.T) - (k0 & ~63) + qrow) * 64 + (k0 & 63) + 4 * g) * 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        floatx4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = s[4 * u + e] / sl2;
+        buffer_store_quad(rsc, x, mine ? at + 32 * u : (int)0x80000000, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m = masked(k0, i) ? m : vmax2(m, s[i]);
+  }
+  m = pair_max32(m);
+  float l = 0.f;
+  floatx16 o[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = zero16();
+  for (int kt = 0; kt + 1 < n_w; ++kt) {
+    floatx16 p = scores(kt * 32);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      p[i] = fast_exp2(p[i] - m);
+      l += p[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float* v = Vb + (int64_t)(kt * 32 + acc_row(i, g)) * L.st;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) o[dt] = mfma_f32(32 * dt + c < L.D ? v[32 * dt + c] : 0.f, p[i], o[dt]);
     }
   }
-  for (int x = 1; x < 64; x *= 2) m = fmaxf(m, xor_shfl(m, x));
-  float l = 0.f, o0 = 0.f, o1 = 0.f;  // d = lane and lane + 64
-  for (int j0 = 0; j0 <= t; j0 += 64) {
-    const float p = fast_exp2(score(j0 + lane) - m);
-    l += j0 + lane <= t ? p : 0.f;
-    for (int x = 0; x < 64 && j0 + x <= t; ++x) {
-      const float px = __shfl(p, x, 64);
-      const float* v = Vb + (int64_t)(j0 + x) * L.st;
-      if (lane < L.D) o0 = fmaf(px, v[lane], o0);
-      if (lane + 64 < L.D) o1 = fmaf(px, v[lane + 64], o1);
+  const int k0 = (n_w - 1) * 32;
+  floatx16 p = scores(k0);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    p[i] = fast_exp2(p[i] - m);
+    l += masked(k0, i) ? 0.f : p[i];
+  }
+#pragma unroll 1
+  for (int x = 0; x < 32 && k0 + x < L.T; ++x) {  // key x = acc_row(i, h)
+    const int i = 4 * (x >> 3) + (x & 3), h = (x >> 2) & 1;
+    float px = p[0];
+#pragma unroll
+    for (int j = 1; j < 16; ++j) px = j == i ? p[j] : px;
+    px = __shfl(px, c + 32 * h, 64);
+    const float* v = Vb + (int64_t)(k0 + x) * L.st;
+    if (k0 + x <= t) {
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int y = 0; y < 16; ++y) {
+          const int d = 32 * dt + acc_row(y, g);
+          if (d < L.D) o[dt][y] = fmaf(px, v[d], o[dt][y]);
+        }
     }
   }
-  for (int x = 1; x < 64; x *= 2) l += xor_shfl(l, x);
-  if (lane < L.D) o[lane] = o0 / l;
-  if (lane + 64 < L.D) o[lane + 64] = o1 / l;
-  if (lse != nullptr && lane == 0) *lse = fmaf(m, kLn2, logf(l));
+  l = pair_sum32(l);
+  if (mine) {
+    store_cols<NDT, VEC>(Ob + (int64_t)qrow * L.st, L.D, g, o, 1.f / l);
+    if (lse != nullptr && g == 0) lse[qrow] = fmaf(m, kLn2, logf(l));
+  }
 }
 
 // SAVE: also keeps the raw scores q.k of every tile it computes in SC (the
@@ -354,11 +432,10 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
     if (LSE != nullptr && g == 0) LSE[(int64_t)bh * L.T + qrow] = fmaf(m, kLn2, logf(l_sum));
   }
   const uint64_t bad = __builtin_amdgcn_ballot_w64(qrow < L.T && !ok);
-  for (uint32_t rows = (uint32_t)(bad | (bad >> 32)); rows != 0; rows &= rows - 1) {
-    const int t = q0 + __builtin_ctz(rows);
-    const int64_t at = base + (int64_t)t * L.st;
-    slow_row<SAVE>(Q + at, Kb, Vb, O + at, LSE == nullptr ? nullptr : LSE + (int64_t)bh * L.T + t, rsc, t, L, sl2,
-                   lane);
+  if (bad != 0) {
+    wait_vmem();  // the kept scores of these rows are written once more
+    again<NKS, NDT, VEC, SAVE>(Q + base, Kb, Vb, O + base, LSE == nullptr ? nullptr : LSE + (int64_t)bh * L.T, rsc, q0,
+                               (uint32_t)(bad | (bad >> 32)), L, sl2, lane);
   }
 }
 
