@@ -77,23 +77,24 @@ struct SplitStage {
   // Sub-stage s of the stage at k0.  VEC: aligned pieces through the operand's
   // buffer descriptor (gemm_vec_ok), k past k_end reading as zero (a lane offset
   // past the descriptor's range; the offset that all lanes share stays on a row
-  // of the operand, K its rows).  Otherwise one predicated load per element.
+  // of the operand, K its rows).  A piece lies in k where the operand is
+  // contiguous along it (K is a multiple of four then), else within one k.
+  // Otherwise one predicated load per element.
   template <bool VEC>
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, const float* p, int64_t s_r, int64_t s_k, int r0,
                                        int R, int k0, int s, int k_end, int K, int tid) {
     const int k = k0 + 4 * s + kpos(tid);
     if (VEC) {
-      const bool past = k >= k_end;  // k_end is a multiple of four, k of KU
       if (KC) {
 #pragma unroll
         for (int u = 0; u < RU; ++u) {
-          const float4 x = buffer_load_quad(rsrc, past ? (int)0x80000000 : off[u], (k0 + 4 * s) * 4);
+          const float4 x = buffer_load_quad(rsrc, k >= k_end ? (int)0x80000000 : off[u], (k0 + 4 * s) * 4);
           v[s][4 * u + 0] = x.x, v[s][4 * u + 1] = x.y, v[s][4 * u + 2] = x.z, v[s][4 * u + 3] = x.w;
         }
       } else {
-        const int vo = past ? (int)0x80000000 : off[0];
 #pragma unroll
         for (int i = 0; i < KU; ++i) {
+          const int vo = k + i >= k_end ? (int)0x80000000 : off[0];
           const int so = (int)(min(k0 + 4 * s + i, K - 1) * s_k * 4);
           if constexpr (RU == 4) {
             const float4 x = buffer_load_quad(rsrc, vo, so);
@@ -350,13 +351,15 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
 namespace {
 
 // 128-bit (row-contiguous operands: 64-bit) buffer loads: every row 16-byte
-// aligned along its operand's contiguous direction (a_vec, b_vec), K % 4 == 0,
-// a row-contiguous operand's extent a multiple of four (its pieces do not
-// straddle the end), and each operand's reachable extent (one batch) below
-// 2 GiB (32-bit offsets).  Otherwise one load per element.
+// aligned along its operand's contiguous direction (a_vec, b_vec), that
+// direction's extent a multiple of four (pieces do not straddle the end), and
+// each operand's reachable extent (one batch) below 2 GiB (32-bit offsets).
+// Otherwise one load per element.  Weight gradients, where both operands are
+// row-contiguous, take any number of positions.
 template <bool A_KC, bool B_KC>
 bool gemm_vec_ok(GemmArgs& g) {
-  if (!(g.a_vec && g.b_vec && g.K % 4 == 0 && (A_KC || g.M % 4 == 0) && (B_KC || g.N % 4 == 0))) return false;
+  if (!(g.a_vec && g.b_vec && ((!A_KC && !B_KC) || g.K % 4 == 0) && (A_KC || g.M % 4 == 0) && (B_KC || g.N % 4 == 0)))
+    return false;
   const int64_t a_ext = 4 * (A_KC ? (int64_t)(g.M - 1) * g.a_sm + g.K : (int64_t)(g.K - 1) * g.a_sk + g.M);
   const int64_t b_ext = 4 * (B_KC ? (int64_t)(g.N - 1) * g.b_sn + g.K : (int64_t)(g.K - 1) * g.b_sk + g.N);
   if (a_ext >= ((int64_t)1 << 31) || b_ext >= ((int64_t)1 << 31)) return false;
