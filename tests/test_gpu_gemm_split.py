@@ -30,8 +30,9 @@ def _check(name, got, a, b, extra=0.0, adds=0):
     print(f"  {name} rel {float((got.double() - ref).norm() / ref.norm()):.2e}", flush=True)
 
 
-# (M, N, K): whole 128-wide tiles, one row / column past them, 64-column and
-# few-column outputs, odd k (unaligned rows), a k remainder of 4, few rows
+# (M, N, K): whole tiles, one row / column past them, 64-column and few-column
+# outputs, odd k (unaligned rows), a k remainder of 4, few rows (mostly 64 x 64
+# tiles; every other instance: INSTANCES)
 SHAPES = [(512, 256, 256), (513, 257, 260), (129, 1025, 132), (4100, 64, 64), (700, 36, 1000), (301, 203, 333),
           (33, 768, 768), (2048, 130, 70), (4100, 513, 260), (8200, 64, 1028)]
 
@@ -53,6 +54,56 @@ def test_linear_pair_within_fp32_bound(pkg, torch_dev, M, N, K, pad):
     dw, db = pkg.linear_bwd_dw(dy, x)
     _check("dw", dw, dy.t().contiguous(), x, adds=32)
     _check("db", db[:, None], dy.t().contiguous(), torch.ones(M, 1, device=dev), adds=M)
+
+
+# One shape for every instance that a call can reach: (entry, M, N, K, tile rows, tile
+# columns, 128-bit loads, split-K).  Rows, columns and k just past whole tiles and stages.
+INSTANCES = [("y", 6001, 517, 36, 128, 128, True, False), ("y", 6001, 517, 133, 128, 128, False, False),
+             ("y", 8193, 129, 36, 128, 64, True, False), ("y", 8193, 129, 133, 128, 64, False, False),
+             ("y", 6001, 129, 36, 64, 128, True, False), ("y", 6001, 129, 133, 64, 128, False, False),
+             ("y", 257, 129, 516, 64, 64, True, False), ("y", 257, 257, 261, 64, 64, False, False),
+             ("dx", 4097, 68, 516, 128, 128, True, False), ("dx", 12289, 65, 132, 128, 128, False, False),
+             ("dx", 6001, 68, 260, 128, 64, True, False), ("dx", 8193, 65, 133, 128, 64, False, False),
+             ("dx", 6001, 68, 132, 64, 128, True, False), ("dx", 6001, 65, 133, 64, 128, False, False),
+             ("dx", 257, 260, 260, 64, 64, True, False), ("dx", 257, 129, 517, 64, 64, False, False),
+             ("dw", 4097, 516, 516, 128, 128, True, True), ("dw", 4097, 517, 516, 128, 128, False, True),
+             ("dw", 4097, 516, 260, 128, 64, True, True), ("dw", 4097, 517, 260, 128, 64, False, True),
+             ("dw", 2049, 516, 516, 64, 128, True, True), ("dw", 4097, 257, 517, 64, 128, False, True),
+             ("dw", 16001, 192, 192, 64, 64, True, True), ("dw", 300, 1028, 2052, 128, 128, True, False),
+             ("dw", 300, 1028, 2049, 128, 128, False, False), ("dw", 513, 1540, 772, 64, 128, True, False),
+             ("dw", 513, 1540, 773, 64, 128, False, False)]
+
+
+@pytest.mark.parametrize("entry,M,N,K,bm,bn,vec,partial", INSTANCES)
+def test_every_instance(pkg, torch_dev, entry, M, N, K, bm, bn, vec, partial):
+    """Each instance of the kernel at partial tiles and a k remainder, and that it is the one that
+    ran; split-K sums repeat bit for bit."""
+    from torch.profiler import ProfilerActivity, profile
+    torch, dev = torch_dev
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x, w, b, dy = rnd(M, K), rnd(N, K), rnd(N), rnd(M, N)
+    call = {"y": lambda: pkg.linear_fwd(x, w, b), "dx": lambda: pkg.linear_bwd_dx(dy, w),
+            "dw": lambda: pkg.linear_bwd_dw(dy, x)}[entry]
+    call()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    ran = [e.name for e in prof.events() if "gemm_split_kernel" in e.name]
+    kc = {"y": "true, true", "dx": "true, false", "dw": "false, false"}[entry]
+    assert len(ran) == 1 and f"gemm_split_kernel<{bm}, {bn}, " in ran[0], ran
+    assert f", {kc}, {str(vec).lower()}, {str(partial).lower()}>" in ran[0], ran
+    if entry == "y":
+        _check("y", out, x, w.t().contiguous(), b.double()[None, :], adds=1)
+    elif entry == "dx":
+        _check("dx", out, dy, w)
+    else:
+        _check("dw", out[0], dy.t().contiguous(), x, adds=32)
+        _check("db", out[1][:, None], dy.t().contiguous(), torch.ones(M, 1, device=dev), adds=M)
+        again = call()
+        assert torch.equal(out[0], again[0]) and torch.equal(out[1], again[1])
 
 
 def beside_a_step(g, kind, *shape):

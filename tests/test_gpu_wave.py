@@ -128,3 +128,29 @@ def test_wave_backward_is_deterministic(pkg, torch_dev, family):
     g2 = pkg.wave_attention_backward_full(W, cache, tdy)
     for k in ("d_normed", "d_harmonic_raw", "d_proj_w", "d_v_w", "out_proj_w"):
         assert torch.equal(getattr(g1, k), getattr(g2, k)), k
+
+
+def test_wide_value_projections(pkg, torch_dev):
+    """Heads of 96 over 1602 positions: the per-head value projections and their input gradient,
+    which is added to the projections', are batched products of more than 2^24 multiply-adds.
+
+    The gradient of a phase atan2(s, r) goes with 1 / |(r, s)|, and so does what rounding r and s
+    (sums of E products of sizes up to 4, error about 4 sqrt(E) 2^-24 = 5e-6 between two orders at
+    most, a tenth of it as a rule) makes of it: rows with a head nearer than 0.1 to the origin are
+    left out of the comparison of d_x."""
+    torch, dev = torch_dev
+    B, T, E, H, C = 2, 801, 480, 5, 16
+    w, x, W, tx = _setup(pkg, torch, dev, B, T, E, H, C, seed=11)
+    dy = (np.random.default_rng(T).normal(size=(B, T, E)) / math.sqrt(B * T)).astype(np.float32)
+    _, _, cache = pkg.wave_attention_forward(W, tx)
+    d_x = pkg.wave_attention_backward_full(W, cache, torch.from_numpy(dy).to(dev)).d_normed.cpu().numpy()
+    phase = cache.phase.cpu().numpy()
+    v_w, v_b = w["v_w"].astype(np.float64), w["v_b"].astype(np.float64)
+    want = np.einsum("bthi,hji->bthj", x.reshape(B, T, H, E // H).astype(np.float64), v_w) + v_b
+    assert_parity("values", cache.values.cpu().numpy().reshape(B, T, H, E // H), want)
+    rs = cache.proj.cpu().numpy().reshape(B, T, H, 2 + C)[..., :2]
+    far = (np.hypot(rs[..., 0], rs[..., 1]) >= 0.1).all(-1)
+    assert far.mean() > 0.9
+    for b in range(B):
+        ref = oracle.wave_bwd(x[b], w, dy[b], "f32", phase_in=phase[b])["d_x"]
+        assert_parity(f"d_x b{b}", d_x[b][far[b]], ref[far[b]])
