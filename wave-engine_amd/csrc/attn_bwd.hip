@@ -676,11 +676,10 @@ __global__ __launch_bounds__(256) WHA_DMA_WPE(DP) void attn_bwd_dkv_dma_kernel(
     const int krow = k0w + lq;
     // K unscaled: the recomputed S is the plain dot product q.k (started from
     // -LSE/scale), and scale*log2(e) is applied once per score in the
-    // exponent.  The forward forms q*(scale*log2(e)) . k, whose rounding is
-    // common to every key of a row and cancels against its LSE; scaling K
-    // here instead would round each key's scores differently from the
-    // forward's, and dQ = dS K amplifies such a per-key mismatch by the size
-    // of K wherever large scores come from a large shared key component.
+    // exponent, as the forward does.  Scaling K here instead would round each
+    // key's scores differently from the forward's, and dQ = dS K amplifies
+    // such a per-key mismatch by the size of K wherever large scores come from
+    // a large shared key component.
     float kf[SAVED ? 1 : DG], vf[DG];
     if constexpr (!SAVED) load_row_frag_dma<DP>(K + base, krow, L.T, L.D, L.st, g, 1.f, kf);
     load_row_frag_dma<DP>(V + base, krow, L.T, L.D, L.st, g, 1.f, vf);

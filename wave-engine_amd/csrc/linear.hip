@@ -43,6 +43,7 @@
 
 namespace wha {
 
+constexpr int kBM = 64;  // output rows per block
 
 // Staging of one ROWS x KT operand tile; element (r, k) of the source is
 // p[r*s_r + k*s_k].  KC (s_k == 1, rows of the tile are source rows): LDS
@@ -177,12 +178,12 @@ struct GemmStage {
 };
 
 // MFMA work of one KT-deep stage held in LDS.
-template <int BM, int KT, int WN, bool A_KC, bool B_KC>
+template <int KT, int WN, bool A_KC, bool B_KC>
 __device__ __forceinline__ void gemm_stage_mfma(const float* As, const float* Bs,
-                                                floatx4 (&acc)[4][BM * WN / 64]) {
-  using SA = GemmStage<BM, KT, A_KC>;
+                                                floatx4 (&acc)[4][WN]) {
+  using SA = GemmStage<kBM, KT, A_KC>;
   using SB = GemmStage<64 * WN, KT, B_KC>;
-  constexpr int MT = BM * WN / 64;  // 16-row m tiles per wave
+  constexpr int MT = WN;  // 16-row m tiles per wave
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int lq = lane & 15, gq = lane >> 4;
   const int wn = wave % WN, wm = wave / WN;
@@ -203,15 +204,15 @@ __device__ __forceinline__ void gemm_stage_mfma(const float* As, const float* Bs
 }
 
 // Bias gradient of the weight-gradient GEMM: the per-thread row sums rs (rows
-// 4*(tid % (BM/4)) .. +3 of the block's A tile) added over the threads in
+// 4*(tid % 16) .. +3 of the block's A tile) added over the threads in
 // increasing tid order through LDS (red: >= 1024 floats, free of other use),
 // written by the blocks of the first column tile.
-template <int BM, bool PARTIAL>
+template <bool PARTIAL>
 __device__ __forceinline__ void gemm_rowsum_store(const GemmArgs& g, const float4& rs, int m0, int bt,
                                                   float* red_lds) {
   if ((PARTIAL ? g.rowsum_part : g.rowsum) == nullptr) return;
   // rows rc..rc+3 (rc = 4*(tid % R4)) are summed by the 256/R4 threads tid % R4 == rc/4
-  constexpr int R4 = BM / 4;
+  constexpr int R4 = kBM / 4;
   const int tid = threadIdx.x;
   float4* red = reinterpret_cast<float4*>(red_lds);
   __syncthreads();
@@ -236,11 +237,11 @@ __device__ __forceinline__ void gemm_rowsum_store(const GemmArgs& g, const float
 }
 
 // Epilogue: acc[nt][mt] of each wave to C (bias, accumulate, split-K partials).
-template <int BM, int WN, bool A_KC, bool B_KC, bool PARTIAL>
-__device__ __forceinline__ void gemm_store(const GemmArgs& g, const floatx4 (&acc)[4][BM * WN / 64], int m0, int n0,
+template <int WN, bool A_KC, bool B_KC, bool PARTIAL>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, const floatx4 (&acc)[4][WN], int m0, int n0,
                                            int bt) {
-  using SA = GemmStage<BM, 16, A_KC>;
-  constexpr int MT = BM * WN / 64;
+  using SA = GemmStage<kBM, 16, A_KC>;
+  constexpr int MT = WN;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int lq = lane & 15, gq = lane >> 4;
   const int wn = wave % WN, wm = wave / WN;
@@ -305,12 +306,12 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& g, const floatx4 (&ac
 // across the MFMA work.  A partial stage at the end of the k range follows on
 // its own.  FA / FB: the block's A / B rows are all in bounds and 16-byte
 // aligned, so their k-full stages load unpredicated.
-template <int BM, int KT, int WN, bool A_KC, bool B_KC, bool FA, bool FB>
+template <int KT, int WN, bool A_KC, bool B_KC, bool FA, bool FB>
 __device__ __forceinline__ void gemm_mainloop(const GemmArgs& g, const float* A,
                                               const float* Bm, int m0, int n0, int k_begin,
                                               int k_end, float* As, float* Bs,
-                                              floatx4 (&acc)[4][BM * WN / 64], float4& rs) {
-  using SA = GemmStage<BM, KT, A_KC>;
+                                              floatx4 (&acc)[4][WN], float4& rs) {
+  using SA = GemmStage<kBM, KT, A_KC>;
   using SB = GemmStage<64 * WN, KT, B_KC>;
   const int tid = threadIdx.x;
   const int nfull = k_end > k_begin ? (k_end - k_begin) / KT : 0;
@@ -333,7 +334,7 @@ __device__ __forceinline__ void gemm_mainloop(const GemmArgs& g, const float* A,
     // merge them with the prologue's into one load after the loop-header phi,
     // right before the LDS store that waits for it.
     asm volatile("" ::: "memory");
-    gemm_stage_mfma<BM, KT, WN, A_KC, B_KC>(As, Bs, acc);
+    gemm_stage_mfma<KT, WN, A_KC, B_KC>(As, Bs, acc);
   }
   const int kp = k_begin + nfull * KT;
   if (kp < k_end) {
@@ -344,19 +345,19 @@ __device__ __forceinline__ void gemm_mainloop(const GemmArgs& g, const float* A,
     sb.store(Bs, tid);
     if (!A_KC) sa.add_to(rs);
     __syncthreads();
-    gemm_stage_mfma<BM, KT, WN, A_KC, B_KC>(As, Bs, acc);
+    gemm_stage_mfma<KT, WN, A_KC, B_KC>(As, Bs, acc);
   }
 }
 
-// BM x 64*WN output tile per 256-thread block, (4/WN) x WN waves of
-// (BM*WN/4) x 64, KT-deep k stages.  MFMA rows are output columns n, MFMA
+// 64 x 64*WN output tile per 256-thread block, (4/WN) x WN waves of
+// 16*WN x 64, KT-deep k stages.  MFMA rows are output columns n, MFMA
 // columns output rows m.
-template <int BM, int KT, int WN, bool A_KC, bool B_KC, bool PARTIAL>
+template <int KT, int WN, bool A_KC, bool B_KC, bool PARTIAL>
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
   constexpr int BN = 64 * WN;
-  using SA = GemmStage<BM, KT, A_KC>;
+  using SA = GemmStage<kBM, KT, A_KC>;
   using SB = GemmStage<BN, KT, B_KC>;
-  constexpr int MT = BM * WN / 64;  // 16-row m tiles per wave
+  constexpr int MT = WN;  // 16-row m tiles per wave
   __shared__ __align__(16) float As[SA::ELEMS];
   __shared__ __align__(16) float Bs[SB::ELEMS];
   // XCD-aware tile order: blocks are dealt round-robin to the 8 XCDs by linear
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
   int tile = (int)(blockIdx.y * gridDim.x + blockIdx.x);
   const int tiles = (int)(gridDim.x * gridDim.y);
   if (tiles % 8 == 0) tile = (tile % 8) * (tiles / 8) + tile / 8;
-  const int n0 = (tile % (int)gridDim.x) * BN, m0 = (tile / (int)gridDim.x) * BM;
+  const int n0 = (tile % (int)gridDim.x) * BN, m0 = (tile / (int)gridDim.x) * kBM;
   const int bt = (int)blockIdx.z / g.splits;
   const int k_begin = ((int)blockIdx.z % g.splits) * g.k_chunk;
   const float* A = g.a + bt * g.a_sb;
@@ -380,21 +381,21 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     for (int j = 0; j < MT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   // Interior blocks take unpredicated loads for every k stage but a partial last one.
-  const bool fa = g.a_vec && m0 + BM <= g.M;
+  const bool fa = g.a_vec && m0 + kBM <= g.M;
   const bool fb = g.b_vec && n0 + BN <= g.N;
   float4 rs = make_float4(0.f, 0.f, 0.f, 0.f);
   if (fa && fb)
-    gemm_mainloop<BM, KT, WN, A_KC, B_KC, true, true>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
+    gemm_mainloop<KT, WN, A_KC, B_KC, true, true>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
   else if (fa)
-    gemm_mainloop<BM, KT, WN, A_KC, B_KC, true, false>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
+    gemm_mainloop<KT, WN, A_KC, B_KC, true, false>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
   else if (fb)
-    gemm_mainloop<BM, KT, WN, A_KC, B_KC, false, true>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
+    gemm_mainloop<KT, WN, A_KC, B_KC, false, true>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
   else
-    gemm_mainloop<BM, KT, WN, A_KC, B_KC, false, false>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
+    gemm_mainloop<KT, WN, A_KC, B_KC, false, false>(g, A, Bm, m0, n0, k_begin, k_end, As, Bs, acc, rs);
 
   static_assert(SA::ELEMS >= 4 * 256, "the row-sum exchange fits in the A stage");
-  if (!A_KC && n0 == 0) gemm_rowsum_store<BM, PARTIAL>(g, rs, m0, bt, As);  // As is free after the k loop
-  gemm_store<BM, WN, A_KC, B_KC, PARTIAL>(g, acc, m0, n0, bt);
+  if (!A_KC && n0 == 0) gemm_rowsum_store<PARTIAL>(g, rs, m0, bt, As);  // As is free after the k loop
+  gemm_store<WN, A_KC, B_KC, PARTIAL>(g, acc, m0, n0, bt);
 }
 
 // ---------------------------------------------------------------- direct-to-LDS stages
@@ -500,14 +501,14 @@ struct DmaStage {
   }
 };
 
-template <int BM, int KT, int WN, bool A_KC, bool B_KC, bool PARTIAL>
+template <int KT, int WN, bool A_KC, bool B_KC, bool PARTIAL>
 __global__ __launch_bounds__(256) void gemm_dma_kernel(GemmArgs g) {
   constexpr int BN = 64 * WN;
-  constexpr int MT = BM * WN / 64;  // 16-row m tiles per wave
-  using DA = DmaStage<BM, KT, A_KC>;
+  constexpr int MT = WN;  // 16-row m tiles per wave
+  using DA = DmaStage<kBM, KT, A_KC>;
   using DB = DmaStage<BN, KT, B_KC>;
-  __shared__ __align__(16) float As0[BM * KT];
-  __shared__ __align__(16) float As1[BM * KT];
+  __shared__ __align__(16) float As0[kBM * KT];
+  __shared__ __align__(16) float As1[kBM * KT];
   __shared__ __align__(16) float Bs0[BN * KT];
   __shared__ __align__(16) float Bs1[BN * KT];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(GemmArgs g) {
   int tile = (int)(blockIdx.y * gridDim.x + blockIdx.x);
   const int tiles = (int)(gridDim.x * gridDim.y);
   if (tiles % 8 == 0) tile = (tile % 8) * (tiles / 8) + tile / 8;
-  const int n0 = (tile % (int)gridDim.x) * BN, m0 = (tile / (int)gridDim.x) * BM;
+  const int n0 = (tile % (int)gridDim.x) * BN, m0 = (tile / (int)gridDim.x) * kBM;
   const int bt = (int)blockIdx.z / g.splits;
   const int k_begin = ((int)blockIdx.z % g.splits) * g.k_chunk;
   const float* A = g.a + bt * g.a_sb;
@@ -546,7 +547,7 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(GemmArgs g) {
   };
   // bias gradient (row-contiguous A, the weight-gradient GEMM): the blocks of
   // the first column tile add up the staged A rows, each thread rows
-  // 4*(tid % (BM/4)) .. +3 over every (256/(BM/4))-th k row of a stage -- the
+  // 4*(tid % 16) .. +3 over every 16th k row of a stage -- the
   // per-thread sums gemm_rowsum_store reduces
   const bool want_rs = !A_KC && n0 == 0 && (PARTIAL ? g.rowsum_part : g.rowsum) != nullptr;
   float4 rs = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -556,11 +557,11 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(GemmArgs g) {
     if (s + 1 < nst) issue(s + 1, An, Bn);
     if constexpr (!A_KC) {
       if (want_rs) {
-        constexpr int R4 = BM / 4, KSTEP = 256 / R4;
+        constexpr int R4 = kBM / 4, KSTEP = 256 / R4;
         const int tid = threadIdx.x;
 #pragma unroll
         for (int kr = tid / R4; kr < KT; kr += KSTEP) {
-          const float4 x = *reinterpret_cast<const float4*>(&Ac[kr * BM + 4 * (tid % R4)]);
+          const float4 x = *reinterpret_cast<const float4*>(&Ac[kr * kBM + 4 * (tid % R4)]);
           rs.x += x.x;
           rs.y += x.y;
           rs.z += x.z;
@@ -589,9 +590,9 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(GemmArgs g) {
     if (s + 1 < nst) step(s + 1, As1, Bs1, As0, Bs0);
   }
 
-  static_assert(BM * KT >= 4 * 256, "the row-sum exchange fits in an A stage");
-  if (!A_KC && n0 == 0) gemm_rowsum_store<BM, PARTIAL>(g, rs, m0, bt, As0);  // after its own barrier
-  gemm_store<BM, WN, A_KC, B_KC, PARTIAL>(g, acc, m0, n0, bt);
+  static_assert(kBM * KT >= 4 * 256, "the row-sum exchange fits in an A stage");
+  if (!A_KC && n0 == 0) gemm_rowsum_store<PARTIAL>(g, rs, m0, bt, As0);  // after its own barrier
+  gemm_store<WN, A_KC, B_KC, PARTIAL>(g, acc, m0, n0, bt);
 }
 
 // C[bt][m][n] (+)= bias[bt][n] + sum_s part[bt*splits + s][m][n], s in increasing order.
@@ -729,9 +730,9 @@ bool gemm_dma_ok(GemmArgs& g) {
   return true;
 }
 
-template <int BM, int KT, int WN, bool A_KC, bool B_KC>
+template <int KT, int WN, bool A_KC, bool B_KC>
 hipError_t gemm_launch(GemmArgs g, float* ws, int splits, const char* name, hipStream_t stream) {
-  const dim3 grid((g.N + 64 * WN - 1) / (64 * WN), (g.M + BM - 1) / BM, splits * g.batch);
+  const dim3 grid((g.N + 64 * WN - 1) / (64 * WN), (g.M + kBM - 1) / kBM, splits * g.batch);
   g.splits = splits;
   const bool dma = gemm_dma_ok<A_KC, B_KC>(g);
   constexpr int KD = WHA_GEMM_DMA_KT;
@@ -739,10 +740,10 @@ hipError_t gemm_launch(GemmArgs g, float* ws, int splits, const char* name, hipS
   if (splits == 1) {
     g.k_chunk = dma ? ((g.K + KD - 1) / KD) * KD : ((g.K + KT - 1) / KT) * KT;
     if (dma) {
-      hipLaunchKernelGGL((gemm_dma_kernel<BM, KD, WN, A_KC, B_KC, false>), grid, dim3(256), 0, stream, g);
+      hipLaunchKernelGGL((gemm_dma_kernel<KD, WN, A_KC, B_KC, false>), grid, dim3(256), 0, stream, g);
       return hipGetLastError();
     }
-    hipLaunchKernelGGL((gemm_kernel<BM, KT, WN, A_KC, B_KC, false>), grid, dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((gemm_kernel<KT, WN, A_KC, B_KC, false>), grid, dim3(256), 0, stream, g);
     return hipGetLastError();
   }
   const int per = (g.K + splits - 1) / splits;
@@ -751,9 +752,9 @@ hipError_t gemm_launch(GemmArgs g, float* ws, int splits, const char* name, hipS
   p.c = ws;
   p.bias = nullptr;
   if (dma)
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, KD, WN, A_KC, B_KC, true>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gemm_dma_kernel<KD, WN, A_KC, B_KC, true>), grid, dim3(256), 0, stream, p);
   else
-    hipLaunchKernelGGL((gemm_kernel<BM, KT, WN, A_KC, B_KC, true>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gemm_kernel<KT, WN, A_KC, B_KC, true>), grid, dim3(256), 0, stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return gemm_reduce(g, ws, stream);
@@ -903,8 +904,8 @@ hipError_t gemm_t(GemmArgs g, float* ws, const char* name, hipStream_t stream, i
   // 128-bit loads need every row start along the contiguous direction 16-byte aligned
   g.a_vec = aligned16(g.a) && g.a_sb % 4 == 0 && (A_KC ? g.a_sm % 4 == 0 : g.a_sk % 4 == 0);
   g.b_vec = aligned16(g.b) && g.b_sb % 4 == 0 && (B_KC ? g.b_sn % 4 == 0 : g.b_sk % 4 == 0);
-  return gemm_bn(g.N) == 64 ? gemm_launch<64, WHA_GEMM_KT, 1, A_KC, B_KC>(g, ws, splits, name, stream)
-                            : gemm_launch<64, WHA_GEMM_KT, 2, A_KC, B_KC>(g, ws, splits, name, stream);
+  return gemm_bn(g.N) == 64 ? gemm_launch<WHA_GEMM_KT, 1, A_KC, B_KC>(g, ws, splits, name, stream)
+                            : gemm_launch<WHA_GEMM_KT, 2, A_KC, B_KC>(g, ws, splits, name, stream);
 }
 
 constexpr int kMaxSplits = 32;

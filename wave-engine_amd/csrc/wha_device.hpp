@@ -355,7 +355,9 @@ __device__ __forceinline__ void buffer_store_float(__amdgpu_buffer_rsrc_t r, flo
 // overwrites them, which this compiler does not always leave: a 128-bit store
 // here came out followed directly by a v_max3_f32 into one of its data
 // registers (the 128-wide kept-scores forward), and the stored scores were
-// wrong in that element.  Stores of 8 bytes have no such hazard.
+// wrong in that element.  Stores of 8 bytes have no such hazard; the optimizer
+// joins two of them again where they end up side by side, so the assembly of
+// every build is scanned for it as well (tests/test_isa_hazards.py).
 __device__ __forceinline__ void buffer_store_quad(__amdgpu_buffer_rsrc_t r, floatx4 v, int voff, int soff) {
   typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
   typedef float floatx2 __attribute__((ext_vector_type(2)));

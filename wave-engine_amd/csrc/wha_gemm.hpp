@@ -22,8 +22,8 @@ struct GemmArgs {
   int splits = 1;      // blockIdx.z = batch index * splits + split index
   int64_t a_sb = 0, b_sb = 0, c_sb = 0, bias_sb = 0;
   bool a_vec = false;  // A's base, batch stride and row stride along its contiguous
-  bool b_vec = false;  // direction are 16-byte multiples (set by gemm_t); same for B
-  // Row sums of A over the k range (A k-contiguous only, i.e. the weight-gradient
+  bool b_vec = false;  // direction are 16-byte multiples (set by gemm_t, gemm_split); same for B
+  // Row sums of A over the k range (A row-contiguous only, i.e. the weight-gradient
   // GEMM, where they are the bias gradient): rowsum[bt*rowsum_sb + m] = sum_k A(m,k),
   // written by the blocks of the first column tile; with split-K each split writes
   // rowsum_part[(bt*splits + split)*M + m] and the reduce adds the splits in order.
@@ -31,7 +31,7 @@ struct GemmArgs {
   int64_t rowsum_sb = 0;
   float* rowsum_part = nullptr;
   // bytes of one batch's A and B that the VEC loads may touch (the buffer
-  // descriptors' extents; set by gemm_vec_ok)
+  // descriptors' extents; set by gemm_dma_ok, gemm_vec_ok)
   uint32_t a_bytes = 0, b_bytes = 0;
 };
 
