@@ -206,7 +206,11 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(GemmArgs g) {
   };
   auto store = [&](int s, unsigned* Ad, unsigned* Bd) {
     sa.store(Ad, s, tid);
-    WHA_FENCE();  // one operand's split at a time: together they spill (128 x 128 weight gradients 137 -> 125 us)
+    // One operand's split at a time: together they take registers from the
+    // loads in flight (M = 4096, us: 128 x 128 weight gradients of 2304 x 768 134.9
+    // -> 122.7, 64 x 128 input gradients of 1280 x 1280 108 -> 97) -- but not in
+    // the 128 x 128 input gradient, where the fence costs (2304 x 768 99 -> 104).
+    if constexpr (!(BM == 128 && BN == 128 && A_KC)) WHA_FENCE();
     sb.store(Bd, s, tid);
   };
   auto multiply = [&](const unsigned* Ac, const unsigned* Bc) {
@@ -435,15 +439,22 @@ GemmPick gemm_pick(int M, int N, int K, int batch, bool rows_contiguous, int max
 // MFMA against split: 1000 x 100 <- 77 forward / dx / dW 8.7 / 8.9 / 21.5
 // against 9.8 / 11.1 / 22.9; above, 1024 x 504 <- 168 13.2 / 14.7 / 13.7
 // against 11.2 / 13.4 / 16.5, 32 x 768 <- 768 32 / 31 / 10.8 against 18 / 20 /
-// 12).
+// 12).  Above, the fp32 kernels are the faster ones by 5-25% (about 1 us) for
+// forwards of at most 256 columns over at most 160 k and for input gradients of
+// at most 256 columns below 2^26 (4312 x 192 <- 128 8.4 against 9.0, dx of 1500 x
+// 192 <- 128 5.7 against 7.8), and by up to 13% for some operands whose rows are
+// not aligned (4001 x 513 <- 512 dx 38.8 against 45.2); the rule leaves those
+// here for the error, a third of the fp32 MFMA's.
 bool gemm_split_ok(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return (double)M * (double)N * (double)K * (double)batch >= (double)(1 << 24);
 }
 // Weight gradients from 2^29 on: below, their few output tiles and the split-K
 // sum set the time (us, fp32 MFMA against split, M x N x K: 1024 x 504 x 168
 // 13.7 / 16.5, 4096 x 504 x 168 19.9 / 20.9, 2048 x 384 x 384 21.2 / 21.1, 12
-// heads of 8192 x 64 x 64 16.1 / 22.7; above, 4096 x 768 x 256 26.5 / 27.7, 1024 x
-// 768 x 768 31.9 / 24.4, 8192 x 216 x 768 47.3 / 39.3).
+// heads of 8192 x 64 x 64 16.1 / 22.7; above, 8192 x 256 x 256 23.0 / 24.0, 4096 x
+// 768 x 256 27.6 / 27.7, 4096 x 384 x 384 32.3 / 24.1, 1024 x 768 x 768 31.9 / 24.4,
+// 8192 x 216 x 768 47.3 / 39.3): the line lies where the smallest outputs are
+// no slower, those of more tiles gain from a little below it.
 bool gemm_split_dw_ok(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return (double)M * (double)N * (double)K * (double)batch >= (double)(1 << 29);
 }
