@@ -17,8 +17,9 @@
  *   - Host entry points take host pointers in the reference's per-sequence
  *     layout and return after the results are in host memory.
  *   - All tensors are fp32, and so is the arithmetic: contractions run on fp32
- *     MFMAs, or on bf16 MFMAs with each fp32 in three exact bf16 parts and six
- *     products accumulated in fp32, whose error is no larger.
+ *     MFMAs, or on bf16 MFMAs with each fp32 in three bf16 parts (exactly) and
+ *     the six products that reach fp32 precision accumulated in fp32: what is
+ *     left out is below one fp32 rounding of each product.
  *   - Entry points are re-entrant and may be called from several host
  *     threads at once (the reference calls the backend from one thread per
  *     batch element, src/cpu/train_loop.rs:320-365).

@@ -28,17 +28,18 @@
 //
 // Forward alone, fp32 MFMA kernel (16 queries per wave, 64 per block) -> this
 // one, us; and the relative error of O against 64 bits:
-//   8 x 12 heads, 1024 x 64       128 -> 87      3.3e-7 -> 1.5e-7
-//   16 x 8 heads, 512 x 48        38.2 -> 29.2   2.7e-7 -> 1.5e-7
-//   4 x 32 heads, 2048 x 128      1074 -> 800    4.5e-7 -> 1.6e-7
-//   3 x 10 heads, 1531 x 56       111 -> 68      3.7e-7 -> 1.6e-7
-//   the same at head dim 50       134 -> 90      4.1e-7 -> 1.4e-7
-//   4 x 16 heads, 700 x 96        101 -> 56      3.4e-7 -> 1.7e-7
-//   8 x 8 heads, 600 x 32         38.0 -> 23.1   2.9e-7 -> 1.3e-7
-//   2 x 32 heads, 333 x 100       41.6 -> 32.5   (fewer blocks than CUs)
-//   1 x 4 heads, 8192 x 64        428 -> 312
-// It was the faster one at every head dim and length tried down to the small
-// problems' limit, so the other is gone.
+//   8 x 12 heads, 1024 x 64       114 -> 77      3.3e-7 -> 1.2e-7
+//   16 x 8 heads, 512 x 48        39.3 -> 27.8   2.7e-7 -> 1.1e-7
+//   4 x 32 heads, 2048 x 128      1071 -> 790    4.4e-7 -> 1.5e-7
+//   3 x 10 heads, 1531 x 56       110 -> 68      3.7e-7 -> 1.3e-7
+//   the same at head dim 50       133 -> 88      4.1e-7 -> 1.6e-7
+//   4 x 16 heads, 700 x 96        100 -> 52      3.3e-7 -> 1.3e-7
+//   8 x 8 heads, 600 x 32         38.1 -> 22.3   2.8e-7 -> 1.0e-7
+//   2 x 32 heads, 333 x 100       41.5 -> 30.7   3.0e-7 -> 1.2e-7 (fewer blocks than CUs)
+//   1 x 4 heads, 8192 x 64        428 -> 300     6.4e-7 -> 1.7e-7
+// and keeping the scores (the figures at `save`): it was the faster one at every
+// head dim and length tried down to the small problems' limit, with and without
+// the scores, so the other is gone.
 #include <type_traits>
 
 #include "wha_launch.hpp"

@@ -9,10 +9,10 @@
 // gemm_reduce sums in a fixed order (deterministic).
 //
 // Bound by the matrix cores and their power: at M = 8192 with N = K = 4096 the
-// kernel runs 200 TFLOP/s of fp32 products (1200 of bf16 ones; MFMA busy 65% at
+// kernel runs 196 TFLOP/s of fp32 products (1180 of bf16 ones; MFMA busy 65% at
 // the 1.75 GHz the card then holds, where a bare loop of bf16 MFMAs on random
-// data reaches 1900) against 141 of the fp32 MFMA kernels; its error against 64
-// bits is a third of theirs (4.0e-7 against 1.1e-6; K = 768 1.7e-7 against
+// data reaches 1900) against 139 of the fp32 MFMA kernels; its error against 64
+// bits is a third of theirs (4.0e-7 against 1.1e-6; K = 768 1.6e-7 against
 // 5.0e-7).
 #include "wha_gemm.hpp"
 #include "wha_split.hpp"
