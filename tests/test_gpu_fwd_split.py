@@ -70,6 +70,38 @@ def test_tile_edges(pkg, T, D):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
 
 
+@pytest.mark.parametrize("D,T,waves", [(68, 33, 2), (80, 64, 2), (80, 65, 2), (96, 127, 2), (96, 129, 2), (72, 256, 2),
+                                       (80, 257, 4), (100, 33, 2), (128, 64, 2), (128, 65, 4), (128, 128, 4),
+                                       (104, 129, 2), (128, 192, 2), (128, 193, 4)])
+def test_short_rows_of_wide_heads(pkg, D, T, waves):
+    """Blocks of two waves (two_waves): tile edges, the kept scores and the gradients from them;
+    the same bits as blocks of four."""
+    from torch.profiler import ProfilerActivity, profile
+    q, k, v = draw(9, 32, T, D, T + D, mixed=True)
+    o, lse = pkg.attn_fwd(q, k, v)
+    torch.cuda.synchronize()
+    sc = pkg.attn_scores_buffer(pkg.layout_of(q), torch.device("cuda:0"))
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        o2, lse2 = pkg.attn_fwd(q, k, v, scores=sc)
+        torch.cuda.synchronize()
+    ran = [e.name for e in prof.events() if "attn_fwd_split_kernel" in e.name]
+    assert len(ran) == 1 and f", {waves}, true, true>" in ran[0], ran
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    check(o, lse, q, k, v, 1 / math.sqrt(D))
+    do = draw(9, 32, T, D, 1)[0]
+    whole = pkg.attn_bwd(q, k, v, o, do, lse, scores=sc)
+    plain = pkg.attn_bwd(q, k, v, o, do, lse)
+    for a, b in zip(whole, plain):
+        assert (a - b).norm() <= 1e-5 * b.norm()
+    # one load per element: always four waves
+    parts = []
+    for x in (q, k, v):
+        buf = torch.empty(x.numel() + 4, device="cuda")
+        parts.append(buf[1:1 + x.numel()].view_as(x).copy_(x))
+    o3, lse3 = pkg.attn_fwd(*parts)
+    assert torch.equal(o, o3) and torch.equal(lse, lse3)
+
+
 def fp32_sums(q, k, v, scale):
     """O and LSE with every sum a chain of fp32 fused multiply-adds (exact in 64 bits, rounded)."""
     T, D = q.shape[-2:]

@@ -2,7 +2,8 @@
 // (wha_split.hpp): o = softmax(q k^T scale, causal) v and the row log-sum-exp,
 // for every problem but the small ones (small_problem).
 //
-// A block takes NW x 32 consecutive queries of one (b,h), a wave 32 of them: Q
+// A block takes NW x 32 consecutive queries of one (b,h) (NW = 4; 2 for short rows
+// of wide heads, two_waves), a wave 32 of them: Q
 // in registers (split, unscaled), 32-key tiles of K and V split by the whole
 // block into two LDS buffers, one barrier per tile -- while a tile is consumed
 // the next one is split into the other buffer and the one after it is loaded.
@@ -37,9 +38,10 @@
 //   8 x 8 heads, 600 x 32         38.1 -> 22.3   2.8e-7 -> 1.0e-7
 //   2 x 32 heads, 333 x 100       41.5 -> 30.7   3.0e-7 -> 1.2e-7 (fewer blocks than CUs)
 //   1 x 4 heads, 8192 x 64        428 -> 300     6.4e-7 -> 1.7e-7
-// and keeping the scores (the figures at `save`): it was the faster one at every
-// head dim and length tried down to the small problems' limit, with and without
-// the scores, so the other is gone.
+// and keeping the scores (the figures at `save`).  It was the faster one at every
+// head dim and length tried but for short rows of many heads (up to 64
+// positions, 192 above head dim 96: the figures at two_waves; 512 heads of 40 x
+// 64 9.0 -> 10.1), so the other, with three times the error, is gone.
 #include <type_traits>
 
 #include "wha_launch.hpp"
@@ -172,7 +174,9 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
     float* __restrict__ LSE, float* __restrict__ SC, View L, float sl2) {
   using T3 = Tile3<NKS, NDT>;
   constexpr int NT = NW * 64, BM = NW * 32;
-  __shared__ __align__(16) unsigned K0[T3::RSIZE], K1[T3::RSIZE], V0[T3::CSIZE], V1[T3::CSIZE];
+  // two waves at the widest head dim: one buffer of V, so that two blocks fit a CU
+  constexpr bool V_TWO = !(NW == 2 && NDT == 4);
+  __shared__ __align__(16) unsigned K0[T3::RSIZE], K1[T3::RSIZE], V0[T3::CSIZE], V1[V_TWO ? T3::CSIZE : 4];
 
   const int BH = L.B * L.H;
   const int n_qt = (L.T + BM - 1) / BM;
@@ -372,7 +376,7 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
     typename decltype(kl)::Pending kw;
     typename decltype(vl)::Pending vw;
     constexpr int PK = decltype(kl)::kPieces, PV = decltype(vl)::kPieces;
-    interleave<NMO, PK + PV + 2>(
+    interleave<NMO, PK + 1 + (V_TWO ? PV + 1 : 0)>(
         [&](auto ic) {
           constexpr int i = decltype(ic)::value, dt = i / 12, e = i % 12;
           if (e == 1) vf[2 * dt + 1] = T3::cols_frag(Vs, dt, 1, lane);
@@ -412,13 +416,22 @@ __global__ __launch_bounds__(NW * 64, NDT <= 2 ? 2 : 1) void attn_fwd_split_kern
     } else {  // every key follows every query of the wave
       store_k(Kst);
       load_k(kt + 3);
-      store_v(Vst);
-      load_v(kt + 2);
+      if constexpr (V_TWO) {
+        store_v(Vst);
+        load_v(kt + 2);
+      }
+    }
+    if constexpr (!V_TWO) {
+      if (kt + 1 < n_kt) {
+        __syncthreads();  // every wave is done with V tile kt
+        store_v(Vst);
+        load_v(kt + 2);
+      }
     }
   };
   for (int kt = 0; kt < n_kt; kt += 2) {
-    step(kt, K1, V0, K0, V1);
-    if (kt + 1 < n_kt) step(kt + 1, K0, V1, K1, V0);
+    step(kt, K1, V0, K0, V_TWO ? V1 : V0);
+    if (kt + 1 < n_kt) step(kt + 1, K0, V_TWO ? V1 : V0, K1, V0);
   }
 
   const float l_sum = pair_sum32(l);
@@ -445,18 +458,30 @@ template <int NKS, int NDT, int NW>
 void fwd_t(const float* q, const float* k, const float* v, float* o, float* lse, float* sc, const View& L, bool vec,
            float sl2, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)((L.T + 32 * NW - 1) / (32 * NW)) * L.B * L.H));
-  if (sc != nullptr && vec)
-    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, true>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
-                       lse, sc, L, sl2);
-  else if (sc != nullptr)
-    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, false, true>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
-                       lse, sc, L, sl2);
-  else if (vec)
-    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, true, false>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
-                       lse, sc, L, sl2);
-  else
-    hipLaunchKernelGGL((attn_fwd_split_kernel<NKS, NDT, NW, false, false>), grid, dim3(64 * NW), 0, stream, q, k, v, o,
-                       lse, sc, L, sl2);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), 0, stream, q, k, v, o, lse, sc, L, sl2);
+  };
+  if constexpr (NW == 4) {  // (two waves: 128-bit loads only)
+    if (!vec)
+      return sc != nullptr ? launch(attn_fwd_split_kernel<NKS, NDT, NW, false, true>)
+                           : launch(attn_fwd_split_kernel<NKS, NDT, NW, false, false>);
+  }
+  sc != nullptr ? launch(attn_fwd_split_kernel<NKS, NDT, NW, true, true>)
+                : launch(attn_fwd_split_kernel<NKS, NDT, NW, true, false>);
+}
+// Head dims above 64, where a CU holds one block of four waves: blocks of two
+// waves (64 queries, two blocks a CU) for short rows that fill more than one
+// round of four-wave blocks -- up to 256 positions, above head dim 96 only
+// where they spare the empty half of a 128-query block.  Kept forward, us, the
+// former fp32 MFMA kernel / four waves / two, at head dim 80: 512 heads of 40
+// 11.7 / 18.4 / 12.4, 352 of 123 27.6 / 28.1 / 26.8, 320 of 130 37.6 / 42.0 /
+// 31.5, 288 of 256 60.0 / 50.8 / 46.6; not 256 of 128 (one round) 20.1 / 16.7 /
+// 17.9, 160 of 384 65.9 / 45.6 / 46.2, 40 of 1000 137 / 72 / 78.  At 128: 512 of
+// 40 13.1 / 23.4 / 16.9, 320 of 130 39.0 / 51.2 / 42.2; not 352 of 123 29.0 /
+// 34.3 / 37.4, 288 of 200 60.8 / 58.6 / 60.8.
+bool two_waves(const View& L) {
+  if ((int64_t)((L.T + 127) / 128) * L.B * L.H <= 256) return false;
+  return L.D <= 96 ? L.T <= 256 : L.T <= 192 && (L.T - 1) % 128 < 64;
 }
 }  // namespace
 
@@ -474,9 +499,11 @@ hipError_t launch_attn_fwd_split(const float* q, const float* k, const float* v,
   else if (L.D <= 64)
     fwd_t<4, 2, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
   else if (L.D <= 96)
-    fwd_t<6, 3, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+    vec && two_waves(L) ? fwd_t<6, 3, 2>(q, k, v, o, lse, sc, L, vec, sl2, stream)
+                         : fwd_t<6, 3, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
   else
-    fwd_t<8, 4, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
+    vec && two_waves(L) ? fwd_t<8, 4, 2>(q, k, v, o, lse, sc, L, vec, sl2, stream)
+                         : fwd_t<8, 4, 4>(q, k, v, o, lse, sc, L, vec, sl2, stream);
   return hipGetLastError();
 }
 
